@@ -823,6 +823,8 @@ stark_qmm_status routed_run(const stark_qmm_routed_args* a, uint8_t* ws, uint64_
     // 17.1 us; 256 experts 21.4 vs 22.6; hidden 1536, 128 experts 37.4 vs
     // 38.3; 256 experts 39.3 vs 49.1)
     const bool one = R == 1 && E <= kOneTokenExperts && (uint64_t)A * H * E <= kOneTokenWork;
+    // prompts on group-64 banks: slots of up to 64 routes (moe_group.hip)
+    const bool wide = R > 16 && a->up.group_size == 64 && a->down.group_size == 64;
     if (one) {
         RouteOneArgs ra{a->router_logits, a->expert_scales, E, A, a->round_weights_bf16, a->round_logits_bf16,
                         (uint32_t)adjust, sort, ids, weights, table, header};
@@ -840,7 +842,7 @@ stark_qmm_status routed_run(const stark_qmm_routed_args* a, uint8_t* ws, uint64_
         void* argv[] = {&g, &ra};
         const uint32_t blocks = padded_items(A, g.tiles, line_tiles(g.tiles, 8));
         QMM_HIP_CHECK(hipLaunchKernel(fn, dim3(blocks), dim3(kWg), argv, 0, stream));
-    } else if (Lw.routes <= kFusedRoutes && R <= kFusedRows && nkeys <= kFusedKeys && nkeys * E <= kFusedCompares) {
+    } else if (!wide && Lw.routes <= kFusedRoutes && R <= kFusedRows && nkeys <= kFusedKeys && nkeys * E <= kFusedCompares) {
         hipLaunchKernelGGL(moe_route_compact, dim3(1), dim3(1024), nkeys * 8, stream, a->router_logits, R, E, A,
                            a->round_weights_bf16, a->round_logits_bf16, a->expert_scales, (uint32_t)adjust, sort,
                            Lw.max_slots, ids, weights, sorted, table, header);
@@ -851,17 +853,30 @@ stark_qmm_status routed_run(const stark_qmm_routed_args* a, uint8_t* ws, uint64_
         if (st != STARK_QMM_OK) return st;
         if (adjust) st = launch_moe_adjust(ids, weights, a->expert_scales, R, E, A, sort, stream);
         if (st != STARK_QMM_OK) return st;
-        hipLaunchKernelGGL(moe_compact, dim3(1), dim3(1024), 0, stream, ids, Lw.routes, E, Lw.max_slots,
-                           slot_routes(R), sorted,
-                           table, header);
-        QMM_HIP_CHECK(hipGetLastError());
+        if (wide) {
+            st = launch_moe_group_slots(ids, Lw.routes, E, sorted, table, header, stream);
+            if (st != STARK_QMM_OK) return st;
+        } else {
+            hipLaunchKernelGGL(moe_compact, dim3(1), dim3(1024), 0, stream, ids, Lw.routes, E, Lw.max_slots,
+                               slot_routes(R), sorted, table, header);
+            QMM_HIP_CHECK(hipGetLastError());
+        }
+    }
+    for (int pass = 0; wide && pass < 2; ++pass) {
+        const bool up = pass == 0;
+        const AffineOp o = up ? bank_op(a->up, E * 2 * H, model, a->input) : bank_op(a->down, E * model, H, act);
+        const MoeGroup g{o.codes, (const uint16_t*)o.scales,
+                         o.corr_kind == STARK_QMM_CORRECTION_BIASES ? (const uint16_t*)o.corr : nullptr,
+                         (const uint16_t*)o.x, up ? act : proj, sorted, table, header, o.os, o.gs, H, model, A, 0};
+        st = launch_moe_group(g, up, sg, Lw.routes, E, stream);
+        if (st != STARK_QMM_OK) return st;
     }
     // 3./4. grouped products, one launch per route-count class in use (the
     // one-token path has run the up product already)
     const int top = (int)count_class(max_count);
     // one token: the down products and the rank accumulation in one launch
     void* down_acc = R == 1 && A <= 8 && model % 16 == 0 ? pick_down_acc_one(H, a->down.group_size) : nullptr;
-    for (int pass = one ? 1 : 0; pass < (down_acc ? 1 : 2); ++pass) {
+    for (int pass = one ? 1 : 0; !wide && pass < (down_acc ? 1 : 2); ++pass) {
         GroupedLaunch g{};
         const bool up = pass == 0;
         g.op = up ? bank_op(a->up, E * 2 * H, model, a->input) : bank_op(a->down, E * model, H, act);

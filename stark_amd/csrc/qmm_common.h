@@ -266,6 +266,25 @@ struct DenseOp {
 };
 stark_qmm_status launch_dense_gemv(const DenseOp& op, hipStream_t stream);
 
+// Grouped expert products of a prompt (moe_group.hip): 4-bit group-64 banks,
+// slots of up to 64 routes of one expert.
+struct MoeGroup {
+    const uint8_t* codes;    // the bank: [experts * rows, K / 2]
+    const uint16_t* scales;  // bf16 planes
+    const uint16_t* corr;    // biases, or NULL (symmetric)
+    const uint16_t* x;       // up: [tokens, model]; down: [routes, hidden]
+    uint16_t* out;           // up: act [routes, hidden]; down: proj [routes, model]
+    const uint32_t* sorted;  // routes in expert order
+    const uint32_t* table;   // slot records: expert, first entry of sorted, count, unused
+    const uint32_t* header;  // [0]: slots
+    uint32_t os, gs;         // plane strides
+    uint32_t hidden, model, active, tiles;
+};
+stark_qmm_status launch_moe_group_slots(const uint32_t* ids, uint32_t routes, uint32_t experts, uint32_t* sorted,
+                                        uint32_t* table, uint32_t* header, hipStream_t stream);
+stark_qmm_status launch_moe_group(MoeGroup g, bool up, bool signed_codes, uint32_t routes, uint32_t experts,
+                                  hipStream_t stream);
+
 // GGUF packed-block matvec (kinds 8 = Q8_0, 12 = Q4_K).
 struct GgufOp {
     const uint8_t* blocks;   // [N, K/block * block_bytes]
