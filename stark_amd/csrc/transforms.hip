@@ -9,12 +9,15 @@
 //    alpha, optional RHT and int8 quantization;
 //  - the output-RHT D-op of the products (kernel.rs:287-300), which runs the
 //    output transform in place on d and adds the bias after it.
-// Work items are one thread each: a 32-value stripe, or a whole scale group
-// (up to four stripes) when quantizing; the butterfly runs in registers in
-// the reference's order (pairs (l, l|s) for s = 1, 2, .., 16), then the
+// A thread owns 8 consecutive values of a row, so every load and store of a
+// wave covers whole lines; four consecutive lanes hold a 32-value stripe and 4,
+// 8 or 16 a scale group. The butterfly runs in the reference's order (pairs
+// (l, l|s) for s = 1, 2, .., 16; distances 8 and 16 through DPP), then the
 // scale 1/sqrt(32) as the reference computes it, so every float matches the
-// CPU restatement. These are small launches (one row of activations per
-// token); the HBM-bound products stay the hot path.
+// CPU restatement. What bounds it is memory for the plain transforms (512 x
+// 4096 bf16 quantized: 58 -> 5 us; one thread per scale group read and wrote
+// strided lines) and the division and expf of each value for the gated ones
+// (512 x 12288 bf16 SiLU, quantized: 169 -> 18 us).
 #include "qmm_common.h"
 
 // The reference evaluates `a * b + c` as a rounded product and a rounded sum;
@@ -32,54 +35,142 @@ __device__ __forceinline__ float rnd(uint32_t dt, float v) {
     return dt == STARK_QMM_BF16 ? bf16_bits_to_f32(f32_to_bf16_bits(v)) : v;
 }
 
-// activation_transform/mod.rs:28-43
-__device__ __forceinline__ void hadamard32(float (&v)[kBlock]) {
+constexpr int kVec = 8;  // values per thread
+
+// 8 values at element i (vec: 16-byte aligned there).
+__device__ __forceinline__ void ld8(const void* p, uint32_t dt, size_t i, bool vec, float (&v)[kVec]) {
+    if (!vec) {
 #pragma unroll
-    for (int s = 1; s < kBlock; s <<= 1)
+        for (int e = 0; e < kVec; ++e) v[e] = ld(p, dt, i + e);
+    } else if (dt == STARK_QMM_F32) {
+        const u32x4 a = *(const u32x4*)((const float*)p + i), b = *(const u32x4*)((const float*)p + i + 4);
 #pragma unroll
-        for (int l = 0; l < kBlock; ++l)
+        for (int e = 0; e < 4; ++e) {
+            v[e] = __uint_as_float(a[e]);
+            v[4 + e] = __uint_as_float(b[e]);
+        }
+    } else {
+        const u32x4 a = *(const u32x4*)((const uint16_t*)p + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[2 * e] = __uint_as_float(a[e] << 16);
+            v[2 * e + 1] = __uint_as_float(a[e] & 0xffff0000u);
+        }
+    }
+}
+
+__device__ __forceinline__ void st8(void* p, uint32_t dt, size_t i, bool vec, const float (&v)[kVec]) {
+    if (!vec) {
+#pragma unroll
+        for (int e = 0; e < kVec; ++e) st(p, dt, i + e, v[e]);
+    } else if (dt == STARK_QMM_F32) {
+        u32x4 a, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            a[e] = __float_as_uint(v[e]);
+            b[e] = __float_as_uint(v[4 + e]);
+        }
+        *(u32x4*)((float*)p + i) = a;
+        *(u32x4*)((float*)p + i + 4) = b;
+    } else {
+        u32x4 a;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = f32_to_bf16_bits(v[2 * e]) | ((uint32_t)f32_to_bf16_bits(v[2 * e + 1]) << 16);
+        *(u32x4*)((uint16_t*)p + i) = a;
+    }
+}
+
+// RHT signs of 8 values (vec: 16-byte aligned there).
+__device__ __forceinline__ void signs8(const int32_t* f, size_t i, bool vec, float (&v)[kVec]) {
+    if (vec) {
+        const u32x4 a = *(const u32x4*)(f + i), b = *(const u32x4*)(f + i + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = (float)(int32_t)a[e];
+            v[4 + e] = (float)(int32_t)b[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < kVec; ++e) v[e] = (float)f[i + e];
+    }
+}
+
+// activation_transform/mod.rs:28-43 over the 32 values of four consecutive
+// lanes (q: this lane's place among them).
+__device__ __forceinline__ void hadamard32(float (&v)[kVec], uint32_t q) {
+#pragma unroll
+    for (int s = 1; s < kVec; s <<= 1)
+#pragma unroll
+        for (int l = 0; l < kVec; ++l)
             if ((l & s) == 0) {
                 const float a = v[l], b = v[l | s];
                 v[l] = a + b;
                 v[l | s] = a - b;
             }
+#pragma unroll
+    for (int l = 0; l < kVec; ++l) {
+        const float o = dpp_f32<DPP_XOR1>(v[l]);  // distance 8
+        v[l] = (q & 1) ? o - v[l] : v[l] + o;
+    }
+#pragma unroll
+    for (int l = 0; l < kVec; ++l) {
+        const float o = dpp_f32<DPP_XOR2>(v[l]);  // distance 16
+        v[l] = (q & 2) ? o - v[l] : v[l] + o;
+    }
     const float scale = 1.0f / __fsqrt_rn((float)kBlock);
 #pragma unroll
-    for (int l = 0; l < kBlock; ++l) v[l] *= scale;
+    for (int l = 0; l < kVec; ++l) v[l] *= scale;
 }
 
-// Int8CodeLayout::index (matmul_a.rs:31-46)
-__device__ __forceinline__ uint32_t code_index(bool grouped, uint32_t i) {
-    if (!grouped) return i;
-    const uint32_t o = i & 7u;
-    return i - o + (o & 1u) * 4u + o / 2u;
+// Sum over 4, 8 or 16 consecutive lanes.
+__device__ __forceinline__ int32_t lanes_sum(int32_t v, uint32_t lanes) {
+    v += (int32_t)dpp_u32<DPP_XOR1>((uint32_t)v);
+    v += (int32_t)dpp_u32<DPP_XOR2>((uint32_t)v);
+    const int32_t v8 = v + (int32_t)dpp_u32<DPP_HALF_MIRROR>((uint32_t)v);
+    const int32_t v16 = v8 + (int32_t)dpp_u32<DPP_MIRROR>((uint32_t)v8);
+    return lanes == 4 ? v : lanes == 8 ? v8 : v16;
 }
 
-// mod.rs:9-26 on one scale group; writes codes (layout order), the scale and
-// the group sums of the sum groups inside it.
-template <int SG>
-__device__ __forceinline__ void quantize_group(const float (&t)[SG], uint32_t base, bool grouped, uint32_t sum_group,
-                                               int8_t* q, float* scale_out, int32_t* sums) {
-    float mn = INFINITY, mx = -INFINITY;
+// mod.rs:9-26 on one scale group of LANES consecutive lanes (this lane: values
+// k .. k + 7 of the row); writes codes (layout order, Int8CodeLayout::index,
+// matmul_a.rs:31-46), the scale and the group sums.
+template <int LANES>
+__device__ __forceinline__ void quantize_group(const float (&t)[kVec], uint32_t k, bool grouped, uint32_t sum_group,
+                                               bool vec, int8_t* q, float* scales, int32_t* sums) {
+    float m = 0.0f;  // the largest |t| that is a number
 #pragma unroll
-    for (int i = 0; i < SG; ++i) {
-        mn = fminf(mn, t[i]);
-        mx = fmaxf(mx, t[i]);
-    }
-    const float m = fmaxf(fabsf(mn), fabsf(mx));
+    for (int i = 0; i < kVec; ++i) m = fmaxf(m, fabsf(t[i]));
+    m = __uint_as_float(group_max<LANES>(__float_as_uint(m)));
     const float divisor = (isfinite(m) && m > 0.0f) ? m / 127.0f : 1.0f;
-    *scale_out = divisor;
+    const uint32_t lane = (k / kVec) % LANES;
+    if (lane == 0) scales[k / (kVec * LANES)] = divisor;
+    int8_t c[kVec];
     int32_t sum = 0;
 #pragma unroll
-    for (int i = 0; i < SG; ++i) {
-        float r = roundf(t[i] / divisor);
-        const int8_t c = isnan(r) ? (int8_t)0 : (int8_t)fminf(fmaxf(r, -127.0f), 127.0f);
-        q[code_index(grouped, base + i)] = c;
-        sum += c;
-        if (sums && ((uint32_t)(i + 1) % sum_group) == 0) {
-            sums[(base + i) / sum_group] = sum;
-            sum = 0;
-        }
+    for (int i = 0; i < kVec; ++i) {
+        const float r = roundf(t[i] / divisor);
+        c[i] = isnan(r) ? (int8_t)0 : (int8_t)fminf(fmaxf(r, -127.0f), 127.0f);
+        sum += c[i];
+    }
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 w = {0, 0};
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        // grouped by nibble: values (0, 2, 4, 6) then (1, 3, 5, 7)
+        const uint32_t b = (uint32_t)(uint8_t)c[i];
+        const int g = (i & 1) * 4 + i / 2;
+        w[g / 4] |= (grouped ? b : 0u) << (8 * (g % 4));
+        w[i / 4] |= (grouped ? 0u : b) << (8 * (i % 4));
+    }
+    if (vec) {
+        *(u32x2*)(q + k) = w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < kVec; ++i) q[k + i] = (int8_t)(w[i / 4] >> (8 * (i % 4)));
+    }
+    if (sums) {
+        const int32_t total = lanes_sum(sum, sum_group / kVec);
+        if (k % sum_group == 0) sums[k / sum_group] = total;
     }
 }
 
@@ -92,45 +183,44 @@ struct TransformArgs {
     int32_t* sums_out;
     const int32_t* factors;
     uint32_t batch, count, op, grouped, scale_group, sum_group, t_dt, bias_dt;
+    uint32_t vec_in, vec_out;  // operands read / results written are aligned for 16-byte (codes 8-byte) access
 };
 
-// ActivationTransform: thread = (row, stripe) for the FP ops, (row, scale group)
-// for the quantizing ops (SG values, SG / 32 stripes).
-template <int SG>
+// ActivationTransform: thread = 8 values; LANES lanes per scale group (4 for the FP ops).
+template <int LANES>
 __global__ __launch_bounds__(256) void activation_transform(TransformArgs a) {
-    const uint32_t per_row = a.count / SG;
+    const uint32_t per_row = a.count / kVec;
     const uint32_t item = blockIdx.x * 256 + threadIdx.x;
     if (item >= a.batch * per_row) return;
-    const uint32_t row = item / per_row, g = item % per_row;
-    const size_t ro = (size_t)row * a.count, k0 = (size_t)g * SG;
+    const uint32_t row = item / per_row, k = item % per_row * kVec;
+    const size_t ro = (size_t)row * a.count;
     const void* src = a.input ? a.input : a.fp_out;
     const bool input_rht = a.op != 1;
-    float t[SG];
+    float v[kVec], f[kVec];
+    ld8(src, a.t_dt, ro + k, a.vec_in, v);
+    signs8(a.factors, k, a.vec_in, f);
+    if (input_rht) {
 #pragma unroll
-    for (int s = 0; s < SG / kBlock; ++s) {
-        float v[kBlock];
+        for (int e = 0; e < kVec; ++e) v[e] *= f[e];
+    }
+    hadamard32(v, item);
+    if (!input_rht) {
 #pragma unroll
-        for (int l = 0; l < kBlock; ++l) {
-            const float x = ld(src, a.t_dt, ro + k0 + s * kBlock + l);
-            v[l] = input_rht ? x * (float)a.factors[k0 + s * kBlock + l] : x;
-        }
-        hadamard32(v);
-#pragma unroll
-        for (int l = 0; l < kBlock; ++l)
-            t[s * kBlock + l] = input_rht ? v[l] : v[l] * (float)a.factors[k0 + s * kBlock + l];
+        for (int e = 0; e < kVec; ++e) v[e] *= f[e];
     }
     if (a.op >= 2) {  // Quantize / QuantizeWithGroupSums
-        quantize_group<SG>(t, (uint32_t)k0, a.grouped != 0, a.sum_group, a.q_out + ro,
-                           a.scales_out + (size_t)row * per_row + g,
-                           a.op == 3 ? a.sums_out + (size_t)row * (a.count / a.sum_group) : nullptr);
+        quantize_group<LANES>(v, k, a.grouped != 0, a.sum_group, a.vec_out, a.q_out + ro,
+                              a.scales_out + (size_t)row * (a.count / a.scale_group),
+                              a.op == 3 ? a.sums_out + (size_t)row * (a.count / a.sum_group) : nullptr);
         return;
     }
+    if (a.bias) {
+        float b[kVec];
+        ld8(a.bias, a.bias_dt, k, a.vec_in, b);
 #pragma unroll
-    for (int i = 0; i < SG; ++i) {
-        float v = t[i];
-        if (a.bias) v = rnd(a.t_dt, v) + ld(a.bias, a.bias_dt, k0 + i);
-        st(a.fp_out, a.t_dt, ro + k0 + i, v);
+        for (int e = 0; e < kVec; ++e) v[e] = rnd(a.t_dt, v[e]) + b[e];
     }
+    st8(a.fp_out, a.t_dt, ro + k, a.vec_out, v);
 }
 
 // ActivationType::activate (gpu_types/activation_type.rs:19-111) on a value
@@ -179,20 +269,10 @@ struct GatedArgs {
     uint32_t gated_dim, batch, value_offset, value_row_stride, act_type, has_alpha;
     float alpha, gate_min, gate_max, value_min, value_max;
     uint32_t clip_gate, clip_value, op, grouped, scale_group, sum_group, t_dt;
+    uint32_t vec_in, vec_out;  // as TransformArgs
 };
 
-__device__ __forceinline__ float gated_one(const GatedArgs& a, size_t batch, uint32_t g) {
-    size_t act_index;
-    float value;
-    if (!a.value) {
-        const size_t base = batch * 2 * a.gated_dim;
-        act_index = base + a.gated_dim + g;
-        value = ld(a.act, a.t_dt, base + g);
-    } else {
-        act_index = batch * a.gated_dim + g;
-        value = ld(a.value, a.t_dt, batch * a.value_row_stride + a.value_offset + g);
-    }
-    float gate = ld(a.act, a.t_dt, act_index);
+__device__ __forceinline__ float gated_one(const GatedArgs& a, float value, float gate) {
     if (a.clip_gate) gate = rnd(a.t_dt, clamp_f(gate, a.gate_min, a.gate_max));
     const bool alpha = a.has_alpha && a.act_type == STARK_QMM_ACT_SILU;
     const float activated = activate(a.act_type, gate, a.t_dt, alpha, a.alpha);
@@ -200,66 +280,136 @@ __device__ __forceinline__ float gated_one(const GatedArgs& a, size_t batch, uin
     return rnd(a.t_dt, value * activated);
 }
 
-// GatedActMul: thread = one element (no RHT), one stripe (RHT, FP out) or one
-// scale group (RHT + quantize).
-template <int SG>
+// First elements of row `batch` of the gate and value operands.
+__device__ __forceinline__ void gated_rows(const GatedArgs& a, size_t batch, const void*& value, size_t& gi, size_t& vi) {
+    value = a.value ? a.value : a.act;
+    gi = a.value ? batch * a.gated_dim : batch * 2 * a.gated_dim + a.gated_dim;
+    vi = a.value ? batch * a.value_row_stride + a.value_offset : batch * 2 * a.gated_dim;
+}
+
+// GatedActMul: thread = 8 values; LANES lanes per scale group when quantizing.
+template <int LANES>
 __global__ __launch_bounds__(256) void gated_act_mul(GatedArgs a) {
-    const uint32_t per_row = a.factors ? a.gated_dim / SG : a.gated_dim;
+    const uint32_t per_row = a.gated_dim / kVec;
     const uint32_t item = blockIdx.x * 256 + threadIdx.x;
     if (item >= a.batch * per_row) return;
     const size_t batch = item / per_row;
-    const uint32_t g = item % per_row;
-    if (!a.factors) {
-        st(a.fp_out, a.t_dt, batch * a.gated_dim + g, gated_one(a, batch, g));
-        return;
-    }
-    const uint32_t k0 = g * SG;
-    float t[SG];
+    const uint32_t k = item % per_row * kVec;
+    const void* value;
+    size_t gi, vi;
+    gated_rows(a, batch, value, gi, vi);
+    float v[kVec], g[kVec];
+    ld8(value, a.t_dt, vi + k, a.vec_in, v);
+    ld8(a.act, a.t_dt, gi + k, a.vec_in, g);
 #pragma unroll
-    for (int s = 0; s < SG / kBlock; ++s) {
-        float v[kBlock];
+    for (int e = 0; e < kVec; ++e) v[e] = gated_one(a, v[e], g[e]);
+    if (a.factors) {
+        signs8(a.factors, k, a.vec_in, g);
 #pragma unroll
-        for (int l = 0; l < kBlock; ++l) {
-            const uint32_t i = k0 + s * kBlock + l;
-            v[l] = gated_one(a, batch, i) * (float)a.factors[i];
-        }
-        hadamard32(v);
-#pragma unroll
-        for (int l = 0; l < kBlock; ++l) t[s * kBlock + l] = v[l];
+        for (int e = 0; e < kVec; ++e) v[e] *= g[e];
+        hadamard32(v, item);
     }
     if (a.op != 0) {
-        const uint32_t spr = a.gated_dim / SG;
-        quantize_group<SG>(t, k0, a.grouped != 0, a.sum_group, a.q_out + batch * a.gated_dim,
-                           a.scales_out + batch * spr + g,
-                           a.op == 2 ? a.sums_out + batch * (a.gated_dim / a.sum_group) : nullptr);
+        quantize_group<LANES>(v, k, a.grouped != 0, a.sum_group, a.vec_out, a.q_out + batch * a.gated_dim,
+                              a.scales_out + batch * (a.gated_dim / a.scale_group),
+                              a.op == 2 ? a.sums_out + batch * (a.gated_dim / a.sum_group) : nullptr);
         return;
     }
-#pragma unroll
-    for (int i = 0; i < SG; ++i) st(a.fp_out, a.t_dt, batch * a.gated_dim + k0 + i, t[i]);
+    st8(a.fp_out, a.t_dt, batch * a.gated_dim + k, a.vec_out, v);
 }
 
+// Rows of no whole number of 8 values (no RHT there): thread = one value.
+__global__ __launch_bounds__(256) void gated_act_mul_one(GatedArgs a) {
+    const uint32_t item = blockIdx.x * 256 + threadIdx.x;
+    if (item >= a.batch * a.gated_dim) return;
+    const size_t batch = item / a.gated_dim;
+    const uint32_t k = item % a.gated_dim;
+    const void* value;
+    size_t gi, vi;
+    gated_rows(a, batch, value, gi, vi);
+    st(a.fp_out, a.t_dt, batch * a.gated_dim + k, gated_one(a, ld(value, a.t_dt, vi + k), ld(a.act, a.t_dt, gi + k)));
+}
+
+// sg: scale group of the quantizing ops, else 32; items: threads.
 template <template <int> class K, class Args>
 stark_qmm_status launch_by_group(uint32_t sg, uint32_t items, const Args& a, hipStream_t stream) {
     if (items == 0) return STARK_QMM_OK;
     const dim3 grid((items + 255) / 256);
     switch (sg) {
-    case 32: hipLaunchKernelGGL(K<32>::fn(), grid, dim3(256), 0, stream, a); break;
-    case 64: hipLaunchKernelGGL(K<64>::fn(), grid, dim3(256), 0, stream, a); break;
-    case 128: hipLaunchKernelGGL(K<128>::fn(), grid, dim3(256), 0, stream, a); break;
+    case 32: hipLaunchKernelGGL(K<4>::fn(), grid, dim3(256), 0, stream, a); break;
+    case 64: hipLaunchKernelGGL(K<8>::fn(), grid, dim3(256), 0, stream, a); break;
+    case 128: hipLaunchKernelGGL(K<16>::fn(), grid, dim3(256), 0, stream, a); break;
     default: return STARK_QMM_INVALID_ARGUMENT;
     }
     QMM_HIP_CHECK(hipGetLastError());
     return STARK_QMM_OK;
 }
 
-template <int SG>
+template <int LANES>
 struct AT {
-    static auto fn() { return activation_transform<SG>; }
+    static auto fn() { return activation_transform<LANES>; }
 };
-template <int SG>
+template <int LANES>
 struct GA {
-    static auto fn() { return gated_act_mul<SG>; }
+    static auto fn() { return gated_act_mul<LANES>; }
 };
+
+bool aligned(const void* p, size_t n) { return ((uintptr_t)p & (n - 1)) == 0; }
+
+// Rows of `width` values: whole rows per launch, so that the items of one stay 32-bit.
+uint32_t rows_per_launch(uint32_t width) { return std::max(1u, 0x7fffffffu / std::max(1u, width)); }
+
+stark_qmm_status run_transform(TransformArgs a, uint32_t sg, hipStream_t stream) {
+    a.vec_in = aligned(a.input ? a.input : a.fp_out, 16) && aligned(a.factors, 16) && aligned(a.bias, 16);
+    a.vec_out = a.op >= 2 ? aligned(a.q_out, 8) : aligned(a.fp_out, 16);
+    const uint32_t rows = a.batch, step = rows_per_launch(a.count);
+    const size_t esz = a.t_dt == STARK_QMM_F32 ? 4 : 2;
+    for (uint32_t r = 0; r < rows; r += step) {
+        TransformArgs b = a;
+        b.batch = std::min(step, rows - r);
+        const size_t e = (size_t)r * a.count;
+        if (a.input) b.input = (const uint8_t*)a.input + e * esz;
+        if (a.fp_out) b.fp_out = (uint8_t*)a.fp_out + e * esz;
+        if (a.q_out) b.q_out = a.q_out + e;
+        if (a.scales_out) b.scales_out = a.scales_out + e / a.scale_group;
+        if (a.sums_out && a.sum_group) b.sums_out = a.sums_out + e / a.sum_group;
+        const stark_qmm_status s = launch_by_group<AT>(sg, b.batch * (a.count / kVec), b, stream);
+        if (s != STARK_QMM_OK) return s;
+        if (rows - r <= step) break;
+    }
+    return STARK_QMM_OK;
+}
+
+stark_qmm_status run_gated(GatedArgs a, uint32_t sg, hipStream_t stream) {
+    const size_t esz = a.t_dt == STARK_QMM_F32 ? 4 : 2;
+    const bool rows8 = a.gated_dim % kVec == 0;
+    a.vec_in = aligned(a.act, 16) && aligned(a.factors, 16) &&
+               (!a.value || (aligned((const uint8_t*)a.value + (size_t)a.value_offset * esz, 16) &&
+                             a.value_row_stride * esz % 16 == 0));
+    a.vec_out = a.op != 0 ? aligned(a.q_out, 8) : aligned(a.fp_out, 16);
+    const uint32_t rows = a.batch, step = rows_per_launch(a.gated_dim);
+    for (uint32_t r = 0; r < rows; r += step) {
+        GatedArgs b = a;
+        b.batch = std::min(step, rows - r);
+        const size_t e = (size_t)r * a.gated_dim;
+        b.act = (const uint8_t*)a.act + e * esz * (a.value ? 1 : 2);
+        if (a.value) b.value = (const uint8_t*)a.value + (size_t)r * a.value_row_stride * esz;
+        if (a.fp_out) b.fp_out = (uint8_t*)a.fp_out + e * esz;
+        if (a.q_out) b.q_out = a.q_out + e;
+        if (a.scales_out) b.scales_out = a.scales_out + e / a.scale_group;
+        if (a.sums_out && a.sum_group) b.sums_out = a.sums_out + e / a.sum_group;
+        if (rows8) {
+            const stark_qmm_status s = launch_by_group<GA>(sg, b.batch * (a.gated_dim / kVec), b, stream);
+            if (s != STARK_QMM_OK) return s;
+        } else {
+            const uint32_t items = b.batch * a.gated_dim;
+            if (items) hipLaunchKernelGGL(gated_act_mul_one, dim3((items + 255) / 256), dim3(256), 0, stream, b);
+            QMM_HIP_CHECK(hipGetLastError());
+        }
+        if (rows - r <= step) break;
+    }
+    return STARK_QMM_OK;
+}
 
 bool float_dt(uint32_t dt) { return dt == STARK_QMM_F32 || dt == STARK_QMM_BF16; }
 
@@ -276,7 +426,8 @@ stark_qmm_status launch_output_rht(void* d, uint32_t d_dt, const void* bias, uin
     a.op = STARK_QMM_TRANSFORM_OUTPUT_RHT;
     a.t_dt = d_dt;
     a.bias_dt = bias_dt;
-    return launch_by_group<AT>(32, rows * (n / 32), a, stream);
+    a.scale_group = kBlock;
+    return run_transform(a, kBlock, stream);
 }
 
 }  // namespace qmm
@@ -323,7 +474,7 @@ stark_qmm_status stark_qmm_activation_transform(const stark_qmm_activation_trans
     a.sum_group = x.sum_group_size;
     a.t_dt = x.data_type;
     a.bias_dt = x.bias_data_type;
-    return launch_by_group<AT>(sg, x.batch_size * (x.element_count / sg), a, (hipStream_t)stream);
+    return run_transform(a, sg, (hipStream_t)stream);
 }
 
 stark_qmm_status stark_qmm_gated_act_mul(const stark_qmm_gated_act_mul_args* args, void* stream) {
@@ -376,8 +527,7 @@ stark_qmm_status stark_qmm_gated_act_mul(const stark_qmm_gated_act_mul_args* arg
     a.scale_group = sg;
     a.sum_group = x.sum_group_size;
     a.t_dt = x.data_type;
-    const uint32_t items = x.batch_dim * (x.hadamard_factors ? x.gated_dim / sg : x.gated_dim);
-    return launch_by_group<GA>(sg, items, a, (hipStream_t)stream);
+    return run_gated(a, sg, (hipStream_t)stream);
 }
 
 }  // extern "C"
