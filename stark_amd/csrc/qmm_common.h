@@ -237,13 +237,26 @@ stark_qmm_status launch_affine_gemm_group(const AffineOp* ops, uint32_t count, i
 // Route adjustment with optional gains (moe.hip).
 stark_qmm_status launch_moe_adjust(uint32_t* ids, float* weights, const float* scales, uint32_t rows,
                                    uint32_t experts, uint32_t active, uint32_t sort_ids, hipStream_t stream);
-// Dense small-M kernel: 4-bit, group 64, M = 3 .. 16, K % 1024 == 0 (qmv_small_m.hip).
+// Dense small-M kernel: 4-bit, group 64, M = 9 .. 16, K % 1024 == 0 (qmv_small_m.hip).
 bool small_m_eligible(const AffineOp* ops, uint32_t count);
+// Whether a launch of these products gives every resident workgroup long runs.
+bool small_m_long(const AffineOp* ops, uint32_t count);
 stark_qmm_status launch_small_m(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream);
 // Skinny dequant product: 4-bit, group 64, M = 17 .. 64, K % 512 == 0, the
 // dequant-GEMM's bf16-effective arithmetic (qgemm_skinny.hip).
 bool skinny_eligible(const AffineOp* ops, uint32_t count);
 stark_qmm_status launch_skinny(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream);
+// Products of 1 to 16 rows, group 64, any K % 64 == 0, N and plane layout (qmv_dense.hip).
+bool dense_eligible(const AffineOp& op, int bits);
+// Which products of one call it takes.
+struct DenseRule {
+    int bits;
+    bool two_rows;  // products of one or two rows
+    bool many_rows;  // 4-bit products of more than eight
+    DenseRule(const AffineOp* ops, uint32_t count, int bits);
+    bool takes(const AffineOp& op) const;
+};
+stark_qmm_status launch_affine_dense(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);
 // Matrix-core kernel for 4/8-bit products with M <= 16 (qmv_mfma.hip).
 bool mfma_eligible(const AffineOp& op, int bits);
 stark_qmm_status launch_affine_mfma(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);

@@ -586,14 +586,23 @@ stark_qmm_status launch_affine_gemv(const AffineOp* ops_in, uint32_t count_in, i
         return e && e[0] == '1';
     }();
     // decode-shaped 4-bit products go to the wave-independent decode kernel
-    std::vector<AffineOp> mfma, decode, others;
+    std::vector<AffineOp> mfma, decode, others, dense;
+    const DenseRule rule(ops_in, count_in, bits);
     for (uint32_t i = 0; i < count_in; ++i) {
         const AffineOp& o = ops_in[i];
+        if (rule.takes(o) && !(force_valu && decode_eligible(o, bits))) {
+            dense.push_back(o);
+            continue;
+        }
         if (mfma_eligible(o, bits) && !(force_valu && decode_eligible(o, bits))) {
             mfma.push_back(o);
             continue;
         }
         (decode_eligible(o, bits) ? decode : others).push_back(o);
+    }
+    if (!dense.empty()) {
+        stark_qmm_status st = launch_affine_dense(dense.data(), (uint32_t)dense.size(), bits, stream);
+        if (st != STARK_QMM_OK) return st;
     }
     if (!mfma.empty()) {
         stark_qmm_status st = launch_affine_mfma(mfma.data(), (uint32_t)mfma.size(), bits, stream);

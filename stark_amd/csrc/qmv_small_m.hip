@@ -320,7 +320,7 @@ __global__ __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(2))) void q
 bool small_m_eligible(const AffineOp* ops, uint32_t count) {
     for (uint32_t i = 0; i < count; ++i) {
         const AffineOp& o = ops[i];
-        if (o.m < 3 || o.m > 16 || o.group_size != 64 || o.k % kSmPass || o.n < (uint32_t)kRows || o.gather)
+        if (o.m < 9 || o.m > 16 || o.group_size != 64 || o.k % kSmPass || o.n < (uint32_t)kRows || o.gather)
             return false;
         if (o.x_dt != STARK_QMM_BF16 || !(o.w_dt == STARK_QMM_BF16 || o.w_dt == STARK_QMM_F16)) return false;
         if (!(o.corr_kind == STARK_QMM_CORRECTION_BIASES || o.corr_kind == STARK_QMM_CORRECTION_SYMMETRIC))
@@ -330,6 +330,22 @@ bool small_m_eligible(const AffineOp* ops, uint32_t count) {
         if ((uint64_t)o.n * o.k / 2 >= (1ull << 31) || (uint64_t)16 * o.k * 2 >= (1ull << 31)) return false;
     }
     return count > 0;
+}
+
+// The dense products' cost that this kernel saves is the activation stage of
+// each 32 rows, through its runs; those need work for many passes per
+// workgroup (16 rows: 11.5 passes per resident workgroup on the Qwen3-8B layer
+// set, 154 us for four layers against 169; 5.9 at hidden 3072 / 8192, 109
+// against 106; 2.2 at hidden 2048 / 6144, 87 against 62).
+bool small_m_long(const AffineOp* ops, uint32_t count) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return false;
+    uint64_t units = 0;
+    for (uint32_t i = 0; i < count; ++i)
+        units += (uint64_t)((ops[i].n + kRows * kSmTiles - 1) / (kRows * kSmTiles)) * (ops[i].k / kSmPass);
+    return units >= 8 * 2 * (uint64_t)cus;
 }
 
 stark_qmm_status launch_small_m(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream) {

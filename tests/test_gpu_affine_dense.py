@@ -1,0 +1,60 @@
+"""Products of 1 to 16 rows, group 64, on the dense kernel: rows and columns at
+the edges of its tiles (4, 8 and 16 rows; 32 columns), K of one group, of one
+chunk and pass and past them, planes that are not 16-byte aligned (7 or 9
+groups a row, odd row counts), corrections, codes, plane and output types and
+D-ops, against the oracle (bar of tests/tolerances.py); batches of several
+products against single ones."""
+import numpy as np
+import pytest
+import torch
+
+from tests import helpers as H
+from tests import test_gpu_affine as A
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 64), (1, 33, 576), (2, 40, 448), (3, 96, 1024), (4, 31, 1088), (5, 64, 2112),
+                                   (8, 100, 3136), (9, 17, 192), (16, 160, 2624)])
+def test_dense_shapes(qmm, oracle, bits, layout, m, n, k):
+    A.run_case(qmm, oracle, m=m, n=n, k=k, bits=bits, gs=64, layout=layout, seed=n + k + m)
+
+
+@pytest.mark.parametrize("correction,signed,w_dt", [(0, False, H.BF16), (1, True, H.F16), (0, True, H.F16)])
+@pytest.mark.parametrize("bits,m", [(4, 3), (4, 12), (8, 7)])
+def test_dense_corrections(qmm, oracle, correction, signed, w_dt, bits, m):
+    A.run_case(qmm, oracle, n=72, k=1216, m=m, bits=bits, gs=64, layout=0, correction=correction, signed=signed, w_dt=w_dt,
+           seed=m)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_dense_d_ops(qmm, oracle, bits):
+    for m, dt in ((2, H.F32), (6, H.BF16), (11, H.F16)):
+        A.run_case(qmm, oracle, m=m, n=45, k=832, bits=bits, ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=4.0,
+                   d_dt=dt, seed=m)
+
+
+@pytest.mark.parametrize("bits,m", [(4, 1), (4, 6), (8, 8), (4, 16)])
+def test_dense_batch_matches_single(qmm, oracle, bits, m):
+    """Five products in one call, of different K and N, some of them another kernel's when alone."""
+    rng = np.random.default_rng(bits + m)
+    kern = qmm.MatmulKernel(H.BF16, H.BF16, H.BF16)
+    args, outs = [], []
+    for n, k in ((200, 704), (33, 704), (64, 2112), (512, 1024), (40, 128)):
+        w = H.affine_weights(oracle, rng, n, k, bits, 64, 1, 1, H.BF16)
+        x = H.to_dev(H.activations(oracle, rng, m, k, H.BF16))
+        b = qmm.QuantizedB(codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), params=qmm.QuantParams(1, n, k // 64),
+                           mode=qmm.MODE_U4 if bits == 4 else qmm.MODE_U8, correction_data=H.to_dev(w["corr"]))
+        for _ in range(2):
+            outs.append(torch.zeros(m * n, dtype=torch.int16, device="cuda"))
+            args.append(qmm.MatmulArguments(a=x, m=m, n=n, k=k, d=outs[-1], b=b))
+    kern.encode_many(args[0::2])
+    for a in args[1::2]:
+        kern.encode_many([a])
+    torch.cuda.synchronize()
+    for a, b in zip(outs[0::2], outs[1::2]):
+        got, want = (H.load(oracle, H.from_dev(t, np.uint16), H.BF16).astype(np.float64) for t in (a, b))
+        # the same kernel gives the same bits; another one another order of the f32 sums (one bf16 ulp)
+        assert np.all(np.abs(got - want) <= 2.0 ** -7 * np.abs(want) + 1e-3 * np.abs(want).max())
