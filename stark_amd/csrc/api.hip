@@ -225,7 +225,7 @@ stark_qmm_status encode_product(stark_qmm_kernel* kr, const stark_qmm_args* args
 bool a8_gemm_entry(const stark_qmm_kernel* kr, const stark_qmm_args* a, AffineOp* op, A8Operand* q, int* bits) {
     const stark_qmm_b& b = a->b;
     if (a->a_kind != STARK_QMM_A_INT8_SYMMETRIC || a->a_code_layout > STARK_QMM_CODES_GROUPED_BY_NIBBLE || !b.codes ||
-        a->d_ops.rht_factors || b.params.materialize_affine_input_sum || a->gather_indices || a->m <= 16 || a->n == 0)
+        a->d_ops.rht_factors || b.params.materialize_affine_input_sum || a->gather_indices || a->m == 0 || a->n == 0)
         return false;
     const uint32_t ag = a->a_scale_group_size, gs = b.group_size;
     if (!(ag == 32 || ag == 64 || ag == 128) || a->k % ag != 0 || !(gs == 32 || gs == 64 || gs == 128) ||
@@ -236,7 +236,7 @@ bool a8_gemm_entry(const stark_qmm_kernel* kr, const stark_qmm_args* a, AffineOp
     if (!a->d || (a->k && (!a->a || !a->a_scales))) return false;
     *q = A8Operand{(const int8_t*)a->a, a->a_scales, a->a_scale_group_size,
                    a->a_code_layout == STARK_QMM_CODES_GROUPED_BY_NIBBLE ? 1u : 0u};
-    return a8_gemm_eligible(*op, *q, *bits);
+    return a8_gemm_eligible(*op, *q, *bits) || a8_dense_eligible(*op, *q, *bits);
 }
 
 }  // namespace

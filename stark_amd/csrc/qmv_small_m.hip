@@ -1,7 +1,6 @@
-// Dense small-M form of the 4-bit MLX-affine product (speculative verify:
-// M = 3 .. 16 activation rows, group size 64, bf16 activations; M = 3 and 4
-// measured 3.18 -> 3.50 TB/s against the slot form on the Qwen3-8B layer set,
-// M = 2 stays on the slot form, 4.18 against 3.61 TB/s here).
+// Dense small-M form of the 4-bit MLX-affine product with runs of tile pairs:
+// 9 to 16 activation rows, group size 64, bf16 activations, launches of many
+// rows of weights (fewer rows, or fewer weights, take qmv_dense; DenseRule).
 //
 // Same arithmetic as the tile engine (mfma_tile.h): codes enter
 // v_mfma_f32_16x16x32_bf16 as raw bf16 bit patterns (p < 256 is p * 2^-133),

@@ -1,0 +1,63 @@
+"""Int8-activation products on the weight-streaming kernel: every workgroup shape
+its rule can choose (rows of 1 to 16, to 32 and more; few and many columns),
+edges of its tiles (rows, 32 to 256 columns) and passes (odd group counts),
+planes of any alignment, both code layouts, activation groups of 64 and 128,
+corrections, codes and D-ops, against the oracle (bar of tests/tolerances.py)."""
+import numpy as np
+import pytest
+import torch
+
+from tests import helpers as H
+from tests.tolerances import check
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(Q, O, m, n, k, bits, ag, grouped, layout, correction=1, signed=False, w_dt=H.BF16, d_dt=H.F32, d_ops=False):
+    rng = np.random.default_rng(m + n + k + bits)
+    w = H.affine_weights(O, rng, n, k, bits, 64, layout, correction, w_dt)
+    q = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    sc = rng.uniform(0.001, 0.1, (m, k // ag)).astype(np.float32)
+    prior = H.store(O, rng.normal(0, 1, m * n).astype(np.float32), d_dt) if d_ops else None
+    bias = H.store(O, rng.normal(0, 0.5, n).astype(np.float32), w_dt) if d_ops else None
+    st, want = O.matmul(a=np.zeros(m * k, np.uint16), m=m, n=n, k=k, codes=w["codes"], scales=w["scales"], correction=correction,
+                        correction_data=w["corr"], layout=layout, row_count=n, group_count=k // 64, bits=bits,
+                        group_size=64, signed_codes=signed, d=prior, ab_scale=0.5 if d_ops else 1.0, accumulate=d_ops,
+                        bias=bias, weights_dt=w_dt, input_dt=H.BF16, output_dt=d_dt, threads=8, a_codes=q.ravel(),
+                        a_scales=sc.ravel(), a_scale_group_size=ag, a_grouped_by_nibble=bool(grouped))
+    assert st == 0
+    d = H.to_dev(prior) if d_ops else torch.zeros(m * n, dtype=torch.float32 if d_dt == H.F32 else torch.int16, device="cuda")
+    a = Q.Int8SymmetricA(values=H.to_dev(q), scales=H.to_dev(sc), scale_group_size=ag,
+                         code_layout=Q.GROUPED_BY_NIBBLE if grouped else Q.SEQUENTIAL)
+    b = Q.QuantizedB(codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), params=Q.QuantParams(layout, n, k // 64),
+                     mode=Q.MODE_U4 if bits == 4 else Q.MODE_U8, correction=correction, signed_codes=signed,
+                     correction_data=None if w["corr"] is None else H.to_dev(w["corr"]))
+    Q.MatmulKernel(w_dt, H.BF16, d_dt).encode(Q.MatmulArguments(
+        a=a, b=b, d=d, m=m, n=n, k=k, d_transform=Q.MatmulDOps(ab_scale=0.5 if d_ops else 1.0, accumulate=d_ops,
+                                                               bias=None if bias is None else H.to_dev(bias))))
+    torch.cuda.synchronize()
+    got = H.load(O, H.from_dev(d, np.float32 if d_dt == H.F32 else np.uint16), d_dt)
+    vals = q.astype(np.float32)[:, [O.int8_code_index(bool(grouped), i) for i in range(k)]] * np.repeat(sc, ag, 1)
+    mag = H.dequant_magnitude(O, w["codes"], w["scales"], w["corr"], n, k, bits, 64, layout, correction, w_dt,
+                              vals.astype(np.float32).ravel(), H.F32, m, signed=signed, out_n=n)
+    check(got, H.load(O, want, d_dt), mag=mag + (4.0 if d_ops else 0.0), label=f"m{m} n{n} k{k} b{bits}")
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("grouped", [0, 1])
+@pytest.mark.parametrize("m,n,k,ag", [(1, 1, 64, 64), (3, 33, 576, 64), (16, 70, 1152, 128), (17, 40, 2112, 64),
+                                      (33, 96, 1280, 128), (20, 16500, 192, 64), (70, 8300, 128, 128),
+                                      (150, 5000, 320, 64)])
+def test_shapes(qmm, oracle, bits, grouped, m, n, k, ag):
+    _run(qmm, oracle, m, n, k, bits, ag, grouped, layout=(m + n) % 2)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("correction,signed,w_dt", [(0, False, H.BF16), (1, True, H.F16), (0, True, H.F16)])
+def test_corrections(qmm, oracle, bits, correction, signed, w_dt):
+    _run(qmm, oracle, 21, 75, 704, bits, 64, 1, 0, correction, signed, w_dt)
+
+
+def test_d_ops(qmm, oracle):
+    _run(qmm, oracle, 5, 45, 832, 4, 64, 1, 1, d_ops=True)
+    _run(qmm, oracle, 40, 300, 832, 8, 64, 0, 1, d_dt=H.BF16, d_ops=True)
