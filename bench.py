@@ -403,8 +403,8 @@ def config1(args, torch, Q):
 
 
 def verify_lines(args, torch, Q, gen, kern, layers, stream):
-    """Config 1 at M = 2, 4, 8, 16 (speculative verify), 32, 64 (short
-    prefill chunks, the skinny dequant product) and 128, 256 (the
+    """Config 1 at M = 2, 4, 8, 16 (speculative verify), 32, 64, 128 (short
+    prefill chunks, the weight-streaming product) and 256 (the
     dequant-GEMM's 128-row tiles): the same layer set and
     rotating copies, M activation rows per product (q/k/v and gate/up share
     theirs), one line each (attached to the default run's line)."""

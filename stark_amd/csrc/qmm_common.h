@@ -234,6 +234,9 @@ bool gemm_eligible(const AffineOp& op, int bits);
 uint32_t gemm_rows(uint32_t k);  // activation rows one dequant-GEMM grid takes at K
 stark_qmm_status launch_affine_gemm(const AffineOp& op, int bits, hipStream_t stream);
 stark_qmm_status launch_affine_gemm_group(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);
+// Weight-streaming kernel for prompts of 17 to 128 rows, group 64 (qgemm_stream.hip).
+bool gemm_stream_eligible(const AffineOp& op, int bits);
+stark_qmm_status launch_gemm_stream(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);
 // Route adjustment with optional gains (moe.hip).
 stark_qmm_status launch_moe_adjust(uint32_t* ids, float* weights, const float* scales, uint32_t rows,
                                    uint32_t experts, uint32_t active, uint32_t sort_ids, hipStream_t stream);
@@ -242,10 +245,6 @@ bool small_m_eligible(const AffineOp* ops, uint32_t count);
 // Whether a launch of these products gives every resident workgroup long runs.
 bool small_m_long(const AffineOp* ops, uint32_t count);
 stark_qmm_status launch_small_m(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream);
-// Skinny dequant product: 4-bit, group 64, M = 17 .. 64, K % 512 == 0, the
-// dequant-GEMM's bf16-effective arithmetic (qgemm_skinny.hip).
-bool skinny_eligible(const AffineOp* ops, uint32_t count);
-stark_qmm_status launch_skinny(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream);
 // Products of 1 to 16 rows, group 64, any K % 64 == 0, N and plane layout (qmv_dense.hip).
 bool dense_eligible(const AffineOp& op, int bits);
 // Which products of one call it takes.

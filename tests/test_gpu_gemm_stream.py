@@ -1,0 +1,58 @@
+"""Prompt products of 17 to 128 rows, group 64, on the weight-streaming kernel:
+rows at the edges of its row blocks (32, 48, 64; one and two blocks), ragged
+columns at both widths (32 and 64 columns a workgroup), K of one group, of a
+pass less one group and past several passes, both plane layouts, corrections,
+codes, plane and output types and D-ops, against the oracle; the weights bit for
+bit; batches against single products."""
+import numpy as np
+import pytest
+import torch
+
+from tests import helpers as H
+from tests import test_gpu_affine as A
+from tests import test_gpu_exact_dequant as E
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits,layout", [(4, 0), (4, 1), (8, 0), (8, 1)])
+@pytest.mark.parametrize("m,n,k", [(17, 1, 64), (32, 33, 192), (33, 40, 320), (48, 97, 576), (49, 31, 1088), (64, 65, 2112),
+                                   (65, 100, 832), (96, 17, 256), (97, 70, 1216), (128, 33, 512)])
+def test_stream_weights_exact(qmm, oracle, bits, layout, m, n, k):
+    E._gemm_exact(qmm, oracle, n=n, k=k, bits=bits, layout=layout, seed=m + n + k, m=m, label="qgemm_stream")
+
+
+@pytest.mark.parametrize("correction,signed", [(0, False), (1, True), (0, True)])
+@pytest.mark.parametrize("bits,m", [(4, 30), (8, 50)])
+def test_stream_corrections_exact(qmm, oracle, correction, signed, bits, m):
+    E._gemm_exact(qmm, oracle, n=72, k=1216, bits=bits, correction=correction, signed=signed, seed=m, m=m, label="qgemm_stream")
+
+
+@pytest.mark.parametrize("m,n,k,f16", [(20, 3000, 448, False), (40, 25000, 320, True), (64, 25000, 192, False),
+                                       (100, 13000, 576, True), (128, 600, 4416, False)])
+def test_stream_sums(qmm, oracle, m, n, k, f16):
+    """Both column widths against the f64 product of the bf16-effective weights, with the D-ops; f16 planes and results at two sizes."""
+    A._skinny_case(qmm, oracle, m, n, k, seed=m + n, ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=30.0,
+                   w_dt=H.F16 if f16 else H.BF16, d_dt=H.BF16 if f16 else H.F32)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_stream_batch_matches_single(qmm, oracle, bits):
+    """Products of different rows, K and N in one call and alone: the same bits."""
+    rng = np.random.default_rng(bits)
+    kern = qmm.MatmulKernel(H.BF16, H.BF16, H.F32)
+    args, outs = [], []
+    for m, n, k in ((17, 200, 704), (48, 33, 704), (64, 13000, 128), (100, 13000, 192), (128, 40, 4416)):
+        w = H.affine_weights(oracle, rng, n, k, bits, 64, 1, 1, H.BF16)
+        x = H.to_dev(H.activations(oracle, rng, m, k, H.BF16))
+        b = qmm.QuantizedB(codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), params=qmm.QuantParams(1, n, k // 64),
+                           mode=qmm.MODE_U4 if bits == 4 else qmm.MODE_U8, correction_data=H.to_dev(w["corr"]))
+        for _ in range(2):
+            outs.append(torch.zeros(m * n, dtype=torch.float32, device="cuda"))
+            args.append(qmm.MatmulArguments(a=x, m=m, n=n, k=k, d=outs[-1], b=b))
+    kern.encode_many(args[0::2])
+    for a in args[1::2]:
+        kern.encode(a)
+    torch.cuda.synchronize()
+    for a, b in zip(outs[0::2], outs[1::2]):
+        assert torch.equal(a, b)
