@@ -26,8 +26,9 @@
 //    issued before its codes, so staging the next chunk leaves the code loads
 //    in flight.
 // Measured (model 2048, hidden 768, 128 experts, top 8, router included): 512
-// tokens 1978 -> 178 us (the products 1103 + 851 -> 86 + 46 us, 4.0 and 2.5
-// TB/s of weights); 30 tokens over 96 experts: the up product 5.2 TB/s. The
+// tokens 1978 -> 178 us, 160 with the router's later product (the products
+// 1103 + 851 -> 86 + 46 us, 4.0 and 2.5 TB/s of weights); 30 tokens over 96
+// experts: the up product 5.2 TB/s. The
 // slot form of mfma_tile.h (16 routes a slot, half of every MFMA empty, codes
 // through LDS, the weights once per 16 routes) stays for group sizes 32 and
 // 128 and for at most 16 tokens.
