@@ -8,8 +8,8 @@
 // registers), dequantises them there and uses them for all of the workgroup's
 // rows (16 MT, at most 64); only the activations go through LDS, copied as they
 // are, [8-value piece in MFMA order][row], double-buffered. The waves' sums meet
-// in LDS at the end. K splits in the same way in every shape, so a row's sum
-// does not depend on the other rows or on what else the launch holds.
+// in LDS at the end. K splits in the same way in every shape, so a sum is the
+// same in each of them.
 // Where the registers allow (PIPE), the operands of the next pass are
 // dequantised beside the matrix products of this one.
 //
@@ -25,7 +25,7 @@
 //     32   29.6 -> 10.2 30.5 -> 11.3 70.3 -> 23.1 62.9 -> 57   218 -> 185
 //     64   32.8 -> 13.5 35.9 -> 15.2 82.1 -> 32.2 84.5 -> 72   340 -> 240
 //    100   22.9 -> 13.8 22.4 -> 21.8 53.5 -> 44   104 -> 100   335 (GEMM)
-//    128   21.0 -> 14.2 20.6 -> 22.1 52.2 -> 46   109 -> 105   352 (GEMM)
+//    128   21.0 -> 14.2 20.6 (GEMM)  52.2 -> 46   109 -> 105   352 (GEMM)
 // 8-bit: 2560/6912 58 -> 26 (17 rows), 61 -> 39 (64), 69 -> 52 (128);
 // 4096/12288 101 -> 63, 105 -> 79, 120 -> 117.
 #include "qmm_common.h"
@@ -289,16 +289,8 @@ stark_qmm_status launch_shape(AffineBatch& b, int bits, hipStream_t stream) {
 
 }  // namespace
 
-// Up to 64 rows every product, and up to 128 those of models of up to 4096
-// columns, whose wider matrices have K <= 4096 (one activation panel of 1 MiB
-// for all workgroups of an XCD's L2) or at most 4096 columns. Above, the GEMM's
-// tiles fill the chip and read the activations half as often: 128 rows of
-// 5120/13824, 5120/17408 and 8192/28672 take 136, 158 and 352 us there against
-// 151, 180 and 416. A few columns of a long K (the k and v of such a model)
-// stay with it too: they come in the launch of the wide products.
 bool gemm_stream_eligible(const AffineOp& o, int bits) {
     if (o.m <= 16 || o.m > 128 || o.group_size != 64 || o.k == 0 || o.k % 64 || o.n == 0 || o.gather) return false;
-    if (o.m > 64 && o.k > 4096 && (o.n > 4096 || o.n < 1280)) return false;
     if ((bits != 4 && bits != 8) || o.x_dt != STARK_QMM_BF16) return false;
     if (!(o.w_dt == STARK_QMM_BF16 || o.w_dt == STARK_QMM_F16)) return false;
     if (!(o.corr_kind == STARK_QMM_CORRECTION_BIASES || o.corr_kind == STARK_QMM_CORRECTION_SYMMETRIC)) return false;
@@ -306,6 +298,28 @@ bool gemm_stream_eligible(const AffineOp& o, int bits) {
     // 32-bit byte offsets
     return (uint64_t)o.n * o.k * bits / 8 < (1ull << 31) && (uint64_t)o.m * o.k * 2 < (1ull << 31) &&
            2 * ((uint64_t)o.n * o.os + (uint64_t)(o.k / 64) * o.gs) < (1ull << 31);
+}
+
+// Whether a launch's products of more than 64 rows run here (all others of up
+// to 64 do). The GEMM then takes what its deepest product's serial K loop
+// takes, about 7.8 ns a value of K, or, with tiles enough, 0.5 us for 2^20
+// weights, where this kernel takes 0.55: here from 62 values of K for 10^6
+// weights. us of a 4-bit layer at 97 rows (values of K for 10^6 weights), GEMM
+// and here: 1024/1024 (176) 13.9 and 10.0, 2560/6912 (99) 53 and 44, 4096/12288
+// (64) 103.5 and 100, 3072/3072 (59) 38.2 and 38.2, 4096/8192 (57) 73.6 and 81.5,
+// 4096/6144 (49) 61.3 and 71.3. Past 112 rows the GEMM's tiles are full and
+// short launches without a deep product stay with it: 128 rows of 1536/1536 (118)
+// 15.6 and 16.9, 2048/2048 (89) 19.3 and 21.2.
+bool gemm_stream_pays(const AffineOp* ops, uint32_t count) {
+    double weights = 0, k = 0;
+    uint32_t m = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (ops[i].m <= 64) continue;
+        weights += 1e-6 * ops[i].n * ops[i].k;
+        k = std::max(k, (double)ops[i].k);
+        m = std::max(m, ops[i].m);
+    }
+    return k >= 62 * weights && (m <= 112 || k >= 2816 || k >= 150 * weights);
 }
 
 // ops: all gemm_stream_eligible for `bits`, of one plane type; longest K first.
