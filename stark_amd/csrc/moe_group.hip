@@ -33,6 +33,7 @@
 // through LDS, the weights once per 16 routes) stays for group sizes 32 and
 // 128 and for at most 16 tokens.
 #include "qmm_common.h"
+#include "code_layout.h"
 
 namespace qmm {
 namespace {
@@ -105,8 +106,8 @@ __device__ __forceinline__ void group_tile(const MoeGroup& L, GroupLds& lds, uin
     const bool live = n0 < N;
     const size_t bank0 = (size_t)expert * (UP ? 2 * L.hidden : L.model);
     const size_t rowA = bank0 + (live ? n0 : 0), rowB = rowA + (UP ? L.hidden : 16);
-    const uint8_t* cpA = L.codes + (rowA + col) * row_bytes + 16 * kq;
-    const uint8_t* cpB = L.codes + (rowB + col) * row_bytes + 16 * kq;
+    const uint8_t* cpA = L.codes + (rowA + col) * row_bytes + code_lane_offset(kq, K);
+    const uint8_t* cpB = L.codes + (rowB + col) * row_bytes + code_lane_offset(kq, K);
 
     // staging: 16-byte piece tid % 16 of rows tid / 16 + 32 i
     constexpr int XI = (MT + 1) / 2;
@@ -141,8 +142,7 @@ __device__ __forceinline__ void group_tile(const MoeGroup& L, GroupLds& lds, uin
         pb = corr[o];
     };
     const auto load_w = [&](uint32_t c, u32x4 (&w)[2]) {
-        const uint32_t k = c * kChunk;
-        const size_t o = k + 32 * kq < K ? k / 2 : 0;  // codes past K are not computed
+        const size_t o = code_chunk_offset(c * kChunk, kq, K);  // codes past K are not computed
         w[0] = *(const u32x4*)(cpA + o);
         w[1] = *(const u32x4*)(cpB + o);
     };

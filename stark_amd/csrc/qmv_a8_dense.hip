@@ -29,6 +29,7 @@
 //   N  4096, K 12288   17.1 16.0   59.5 15.2  230.0 24.2  229.7  56.9  229.9  96.2
 //   N  7424, K  1920    6.8  7.5   24.2  7.1   46.7  9.8   40.2  23.1   40.9  35.8
 #include "qmm_common.h"
+#include "code_layout.h"
 
 
 namespace qmm {
@@ -118,9 +119,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const uint32_t k = p * kPass + kw * 128;
 #pragma unroll
         for (int h = 0; h < WL; ++h) {
-            // 4-bit: 32 codes at k + 32 kq; 8-bit: 16 codes at k + 64 h + 16 kq (past K: not computed)
-            const uint32_t kl = BITS == 4 ? k + 32 * kq : k + 64 * h + 16 * kq;
-            const size_t o = kl < K ? (size_t)kl * BITS / 8 : 0;
+            const uint32_t o = code_offset<BITS>(k, h, kq, K);
             w[0][h] = *(const u32x4*)(cp[0] + o);
             w[1][h] = *(const u32x4*)(cp[1] + o);
         }

@@ -20,6 +20,7 @@
 // occupy one (two) of a lane's four accumulator entries and only those are
 // scaled (EM = 1, 2, 4 entries).
 #include "qmm_common.h"
+#include "code_layout.h"
 
 namespace qmm {
 namespace {
@@ -118,9 +119,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 
         const uint32_t k = p * kPass + wave * kChunk;
 #pragma unroll
         for (int h = 0; h < WL; ++h) {
-            // 4-bit: 32 codes at k + 32 kq; 8-bit: 16 codes at k + 64 h + 16 kq (past K: not computed)
-            const uint32_t kl = BITS == 4 ? k + 32 * kq : k + 64 * h + 16 * kq;
-            const size_t o = kl < K ? (size_t)kl * BITS / 8 : 0;
+            const uint32_t o = code_offset<BITS>(k, h, kq, K);
             // cached: two waves read the halves of a line (with the
             // nontemporal hint 4-bit rows ran 5% and rows of no whole
             // number of lines up to 20% slower)
