@@ -37,7 +37,7 @@ __device__ __forceinline__ float rnd(uint32_t dt, float v) {
 
 constexpr int kVec = 8;  // values per thread
 
-// 8 values at element i (vec: 16-byte aligned there).
+// 8 f32 or bf16 values at element i (vec: 16-byte aligned there).
 __device__ __forceinline__ void ld8(const void* p, uint32_t dt, size_t i, bool vec, float (&v)[kVec]) {
     if (!vec) {
 #pragma unroll
@@ -57,6 +57,11 @@ __device__ __forceinline__ void ld8(const void* p, uint32_t dt, size_t i, bool v
             v[2 * e + 1] = __uint_as_float(a[e] & 0xffff0000u);
         }
     }
+}
+
+// The same of a bias, which has the plane type of its product and so may be f16 too.
+__device__ __forceinline__ void bias8(const void* p, uint32_t dt, size_t i, bool vec, float (&v)[kVec]) {
+    ld8(p, dt, i, vec && dt != STARK_QMM_F16, v);
 }
 
 __device__ __forceinline__ void st8(void* p, uint32_t dt, size_t i, bool vec, const float (&v)[kVec]) {
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(256) void activation_transform(TransformArgs a) {
     }
     if (a.bias) {
         float b[kVec];
-        ld8(a.bias, a.bias_dt, k, a.vec_in, b);
+        bias8(a.bias, a.bias_dt, k, a.vec_in, b);
 #pragma unroll
         for (int e = 0; e < kVec; ++e) v[e] = rnd(a.t_dt, v[e]) + b[e];
     }

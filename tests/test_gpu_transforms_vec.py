@@ -1,6 +1,7 @@
 """Activation transforms and gated activations (8 values per thread): operands
 that are not 16-byte aligned, rows of no whole number of 8 values, and in-place
-rows, against the oracle bit for bit (identity gate, so no device libm)."""
+rows, against the oracle bit for bit (identity gate, so no device libm); biases of
+every plane type after a product's output RHT."""
 import numpy as np
 import pytest
 import torch
@@ -57,6 +58,43 @@ def test_output_rht_alignment(qmm, oracle, dt, shift):
                                                                                 batch, count)
     torch.cuda.synchronize()
     assert np.array_equal(_bits(d), np.asarray(want).view(np.uint8))
+
+
+@pytest.mark.parametrize("w_dt", [F32, H.F16, BF16])
+@pytest.mark.parametrize("d_dt", [F32, BF16])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("family", ["affine", "dense", "a8"])
+def test_product_rht_bias_types(qmm, oracle, family, shift, d_dt, w_dt):
+    """The bias after a product's output RHT has the type of the planes: the
+    result is the one without a bias (as stored) plus the bias, whatever its
+    type and alignment."""
+    rng = np.random.default_rng(shift + d_dt + w_dt)
+    m, n, k = 3, 64, 128
+    f = H.to_dev(rng.choice([-1, 1], n).astype(np.int32))
+    bias = H.store(oracle, rng.normal(0, 1, n).astype(np.float32), w_dt)
+    x = H.to_dev(H.activations(oracle, rng, m, k, BF16))
+    if family == "dense":
+        b = qmm.FullPrecisionB(values=H.to_dev(H.store(oracle, rng.normal(0, 0.1, n * k).astype(np.float32), w_dt)))
+    else:
+        w = H.affine_weights(oracle, rng, n, k, 4, 64, 1, 1, w_dt)
+        b = qmm.QuantizedB(codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), params=qmm.QuantParams(1, n, k // 64),
+                           correction_data=H.to_dev(w["corr"]))
+    if family == "a8":
+        x = qmm.Int8SymmetricA(values=H.to_dev(rng.integers(-127, 128, (m, k)).astype(np.int8)),
+                               scales=H.to_dev(rng.uniform(0.01, 0.1, (m, k // 64)).astype(np.float32)),
+                               scale_group_size=64, code_layout=qmm.SEQUENTIAL)
+    kern = qmm.MatmulKernel(w_dt, BF16, d_dt)
+
+    def run(bias):
+        d = torch.zeros(m * n, dtype=torch.float32 if d_dt == F32 else torch.int16, device="cuda")
+        kern.encode(qmm.MatmulArguments(a=x, b=b, d=d, m=m, n=n, k=k,
+                                        d_transform=qmm.MatmulDOps(rht_factors=f, bias=bias)))
+        torch.cuda.synchronize()
+        return d
+
+    plain = H.load(oracle, H.from_dev(run(None), np.float32 if d_dt == F32 else np.uint16), d_dt).astype(np.float32)
+    want = H.store(oracle, plain + np.tile(H.load(oracle, bias, w_dt).astype(np.float32), m), d_dt)
+    assert np.array_equal(_bits(run(_shifted(bias, shift))), np.asarray(want).view(np.uint8))
 
 
 @pytest.mark.parametrize("dt", [F32, BF16])
