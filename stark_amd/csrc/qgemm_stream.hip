@@ -295,14 +295,20 @@ bool gemm_stream_eligible(const AffineOp& o, int bits) {
     if (!(o.w_dt == STARK_QMM_BF16 || o.w_dt == STARK_QMM_F16)) return false;
     if (!(o.corr_kind == STARK_QMM_CORRECTION_BIASES || o.corr_kind == STARK_QMM_CORRECTION_SYMMETRIC)) return false;
     if (((uintptr_t)o.codes | (uintptr_t)o.x) & 15) return false;
-    // 32-bit byte offsets
-    return (uint64_t)o.n * o.k * bits / 8 < (1ull << 31) && (uint64_t)o.m * o.k * 2 < (1ull << 31) &&
-           2 * ((uint64_t)o.n * o.os + (uint64_t)(o.k / 64) * o.gs) < (1ull << 31);
+    // 32-bit byte offsets of the planes
+    if (2 * ((uint64_t)o.n * o.os + (uint64_t)(o.k / 64) * o.gs) >= (1ull << 31)) return false;
+    // Weights are rounded to bf16 here, so nothing may come from the kernels
+    // that keep them in f32: besides the GEMM's own products (whose bound on the
+    // codes has 128 rows to spare) only 4-bit ones of up to 64 rows and whole
+    // 512-value steps, which have had bf16 weights up to 2 GiB of codes.
+    return gemm_eligible(o, bits) ||
+           (bits == 4 && o.m <= 64 && o.n >= 16 && o.k % 512 == 0 && (uint64_t)o.n * o.k / 2 < (1ull << 31) &&
+            (uint64_t)64 * o.k * 2 < (1ull << 31));
 }
 
-// Whether a launch's products of more than 64 rows run here (all others of up
-// to 64 do). The GEMM then takes what its deepest product's serial K loop
-// takes, about 7.8 ns a value of K, or, with tiles enough, 0.5 us for 2^20
+// Whether a launch's products of more than 64 rows (all of them gemm_eligible)
+// run here; those of up to 64 always do. The GEMM then takes what its deepest
+// product's serial K loop takes, about 7.8 ns a value of K, or, with tiles enough, 0.5 us for 2^20
 // weights, where this kernel takes 0.55: here from 62 values of K for 10^6
 // weights. us of a 4-bit layer at 97 rows (values of K for 10^6 weights), GEMM
 // and here: 1024/1024 (176) 13.9 and 10.0, 2560/6912 (99) 53 and 44, 4096/12288

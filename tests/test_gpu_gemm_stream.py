@@ -56,3 +56,30 @@ def test_stream_batch_matches_single(qmm, oracle, bits):
     torch.cuda.synchronize()
     for a, b in zip(outs[0::2], outs[1::2]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n,k,m", [(262100, 8192, 17), (40, 4194304 + 64, 32)])
+def test_products_past_the_gemm_keep_f32_weights(qmm, n, k, m):
+    """8-bit products that the GEMM's 32-bit offsets refuse (the last 128 rows
+    below 2 GiB of codes; K past its activation rows) run on the kernels that
+    keep the dequantized weights in f32, whatever their row count: bf16 weights
+    would be 1.6e-3 off the 64-bit product, f32 ones and sums are below 1e-5."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    codes = torch.randint(0, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+    s = (0.002 + 0.002 * torch.rand(n, k // 64, generator=g, device="cuda")).to(torch.bfloat16)
+    b = (-128.0 * s.float() + 0.02 * torch.rand(n, k // 64, generator=g, device="cuda")).to(torch.bfloat16)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    d = torch.zeros(m, n, device="cuda")
+    weights = qmm.QuantizedB(codes=codes, scales=s, correction_data=b, mode=qmm.MODE_U8,
+                             params=qmm.QuantParams(qmm.OUTPUT_GROUP, n, k // 64))
+    args = qmm.MatmulArguments(a=x, b=weights, d=d, m=m, n=n, k=k)
+    kern = qmm.MatmulKernel(H.BF16, H.BF16, H.F32)
+    for call in (lambda: kern.encode(args), lambda: kern.encode_many([args])):
+        d.zero_()
+        call()
+        torch.cuda.synchronize()
+        for r in (0, n - min(n, 64)):
+            rows = slice(r, min(r + 64, n))
+            w = codes[rows].double().view(-1, k // 64, 64) * s[rows].double().unsqueeze(2) + b[rows].double().unsqueeze(2)
+            want = x.double() @ w.view(-1, k).t().contiguous()
+            assert ((d[:, rows].double() - want).norm() / want.norm()).item() < 1e-5
