@@ -2,10 +2,15 @@
 // group 64 and activation groups of 64 or 128: the weights stream from global
 // memory straight into the B operand and only the activations go through LDS.
 //
-// Per 64-value group  acc += (s_a * s) * C + (s_a * sum q_a) * bias_term,
-// C = sum q_a q_w exact in one v_mfma_i32_16x16x64_i8 (8-bit codes enter as
-// q - 128, with 128 s added to the bias term), the bias terms of a chunk's two
-// groups as one v_mfma_f32_16x16x4_f32, as the arithmetic of qgemm_a8.
+// Per 64-value group  acc += s_a * (s * C + sum q_a * bias_term), C = sum q_a q_w
+// exact in one v_mfma_i32_16x16x64_i8. More than 16 rows: as qgemm_a8, the terms
+// (s_a * s) * C and, with a chunk's two groups in one v_mfma_f32_16x16x4_f32,
+// (s_a * sum q_a) * bias_term; 8-bit codes enter as q - 128, with 128 s added to
+// the bias term. Up to 16 rows (they ran on qmv_a8, whose 64 partial sums a row
+// round less than eight waves' in that form, 0.7-0.9e-7 from the 64-bit product
+// against 1.2-1.9e-7): 4-bit codes are centred too (as 16 (q - 8), from the same
+// two masks; the bias term is then small), a group's two terms are added before
+// they join the sum, and the chunk's two groups have a sum each: 0.6-0.9e-7.
 //
 // A lane loads 16 bytes of its weight row. For 4-bit codes these are 32 values
 // and v_permlane32_swap sorts the words so that all four lane groups of an
@@ -23,14 +28,15 @@
 // weights (one row, N 24576, K 4096: 3.7 TB/s); at many the scaling, three
 // vector operations per output and group (conversion, product of the scales,
 // fma) against 16 cycles of matrix work per 16 x 16 x 64.
-// Measured, us before and now (before: qmv_a8 up to 16 rows, qgemm_a8's 128 x 128 tiles above):
-//   rows                    1         16          64         256         512
-//   N 24576, K  4096   28.7 15.6  104.8 15.8   86.0 37.5  105.0 100.8  147.6 (159)
-//   N  4096, K 12288   17.1 16.0   59.5 15.2  230.0 24.2  229.7  56.9  229.9  96.2
-//   N  7424, K  1920    6.8  7.5   24.2  7.1   46.7  9.8   40.2  23.1   40.9  35.8
+// Measured, us before and now (before: qmv_a8 up to 16 rows, qgemm_a8's 128 x 128
+// tiles above; 4-bit, replays of a graph over copies of the weights):
+//   rows                    1          16         64          256         512
+//   N 24576, K  4096   27.4 17.9  93.8 17.6   86.4 36.8  100.3 94.6  134.8 (GEMM)
+//   N  4096, K 12288   15.9 15.2  58.0 16.1  232.2 25.4  230.1 56.0  230.3 93.7
+//   N  7424, K  1920    7.1  5.5  23.8  5.5   47.0 10.2   40.2 22.6   41.0 35.4
+// (in the int8 MLP of 512 rows, between other kernels, the second one takes 108.7.)
 #include "qmm_common.h"
 #include "code_layout.h"
-
 
 namespace qmm {
 namespace {
@@ -50,7 +56,7 @@ struct A8Lds {
         float red[KW > 1 ? KW * R * kCols : 1];  // the K waves' sums, [wave][row][column]
     };
     alignas(16) float sa[2][2 * KW][R];  // activation scale per group and row
-    float ur[2][2 * KW][R];              // activation scale * sum of the group's codes
+    alignas(16) float ur[2][2 * KW][R];  // sum of the group's codes; more than 16 rows: times the scale
     uint32_t pl[2][kThreads];            // raw scale | bias << 16, [group][column]
 };
 
@@ -79,7 +85,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const uint32_t passes = (K + kPass - 1) / kPass;
     const size_t row_bytes = (size_t)K * BITS / 8;
     const bool biased = op.corr_kind == STARK_QMM_CORRECTION_BIASES, sg = (op.flags & FLAG_SIGNED) != 0;
-    const uint32_t flip = BITS == 4 ? (sg ? 0x88888888u : 0u) : (sg ? 0u : 0x80808080u);
+    constexpr bool kFew = MT == 1;            // at most 16 rows
+    constexpr bool kCentred = kFew || BITS == 8;  // codes enter less 2^(BITS - 1), 4-bit ones times 16
+    const uint32_t flip = BITS == 4 ? (sg != kCentred ? 0x88888888u : 0u) : (sg ? 0u : 0x80808080u);
     // activation codes are staged in the order the weights' bytes come in
     const bool permute = BITS == 4 ? ao.grouped == 0 : ao.grouped != 0;
 
@@ -147,15 +155,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             sum += (int)dpp_u32<DPP_XOR2>((uint32_t)sum);
             if (j == 0) {
                 lds.sa[buf][piece >> 2][r] = sv[i];
-                lds.ur[buf][piece >> 2][r] = sv[i] * (float)sum;
+                lds.ur[buf][piece >> 2][r] = kFew ? (float)sum : sv[i] * (float)sum;
             }
         }
         lds.pl[buf][pg * kCols + pc] = ps | (pb << 16);
     };
 
-    f32x4 acc[MT][2];
+    f32x4 acc[MT][2], odd[2];  // odd (at most 16 rows): the sums of the chunks' second groups
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = f32x4{0, 0, 0, 0};
+    odd[0] = odd[1] = f32x4{0, 0, 0, 0};
     const auto compute = [&](int buf, u32x4 (&w)[2][WL], uint32_t ng) {
         if (ng == 0) return;
         const uint32_t* pl = &lds.pl[buf][2 * kw * kCols + 32 * nw + col];
@@ -168,7 +177,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     const uint32_t a = s0[g] ^ flip, c = s1[g] ^ flip;
-                    b[t][g] = u32x4{a & 0x0F0F0F0Fu, (a >> 4) & 0x0F0F0F0Fu, c & 0x0F0F0F0Fu, (c >> 4) & 0x0F0F0F0Fu};
+                    if (kFew) b[t][g] = u32x4{(a << 4) & 0xF0F0F0F0u, a & 0xF0F0F0F0u, (c << 4) & 0xF0F0F0F0u, c & 0xF0F0F0F0u};
+                    else b[t][g] = u32x4{a & 0x0F0F0F0Fu, (a >> 4) & 0x0F0F0F0Fu, c & 0x0F0F0F0Fu, (c >> 4) & 0x0F0F0F0Fu};
                 }
             } else {
 #pragma unroll
@@ -176,6 +186,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
                     for (int q = 0; q < 4; ++q) b[t][g][q] = w[t][g % WL][q] ^ flip;
             }
+        }
+        if constexpr (kFew) {
+            constexpr float unit = BITS == 4 ? 0.0625f : 1.0f, mid = (float)(1 << (BITS - 1));
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                if ((uint32_t)g >= ng) break;
+                const i32x4 a = __builtin_bit_cast(i32x4, lds.xa[buf][(8 * kw + 4 * g + kq) * RP + col]);
+                const f32x4 sa = *(const f32x4*)&lds.sa[buf][2 * kw + g][4 * kq];
+                const f32x4 us = *(const f32x4*)&lds.ur[buf][2 * kw + g][4 * kq];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint32_t q = pl[g * kCols + 16 * t];
+                    const float s = BF ? __uint_as_float(q << 16) : f16_bits_to_f32(q & 0xffffu);
+                    const float bi = BF ? __uint_as_float(q & 0xffff0000u) : f16_bits_to_f32(q >> 16);
+                    const float bt = biased ? fmaf(mid, s, bi) : 0.0f, sc = unit * s;
+                    const i32x4 c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, __builtin_bit_cast(i32x4, b[t][g]),
+                                                                         i32x4{0, 0, 0, 0}, 0, 0, 0);
+                    f32x4& to = g == 0 ? acc[0][t] : odd[t];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) to[e] = fmaf(sa[e], fmaf(sc, (float)c[e], bt * us[e]), to[e]);
+                    asm volatile("" : "+v"(to));
+                }
+            }
+            return;
         }
         // (group by group: with both groups' products in flight the register
         // budget of two workgroups per CU spills, 24 -> 31 us at 32 rows)
@@ -279,6 +313,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 for (int t = 0; t < 2; ++t)
                     store(16 * m + 4 * kq + e, n0 + 32 * nw + 16 * t + col, acc[m][t][e]);
     } else {
+        if (kFew) {
+            acc[0][0] += odd[0];
+            acc[0][1] += odd[1];
+        }
         lds_barrier();  // the activations are read: their LDS takes the sums
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -360,9 +398,12 @@ stark_qmm_status launch_a8_dense(const AffineOp* ops, const A8Operand* as, uint3
     int dev = 0, cus = 0;
     QMM_HIP_CHECK(hipGetDevice(&dev));
     QMM_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    uint32_t rows = 0;
+    for (uint32_t i = 0; i < count; ++i) rows = std::max(rows, ops[i].m);
+    // up to 16 rows the first shape, whose sums are the most exact ones
     int best = 0;
     double cost = 0;
-    for (int i = 0; i < kShapeCount; ++i) {
+    for (int i = 0; i < (rows <= 16 ? 1 : kShapeCount); ++i) {
         const double c = shape_cost(kShapes[i], ops, count, (uint32_t)std::max(cus, 1));
         if (i == 0 || c < cost) {
             best = i;
