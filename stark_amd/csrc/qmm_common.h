@@ -340,7 +340,7 @@ struct A8Batch {
 bool a8_gemm_eligible(const AffineOp& op, const A8Operand& a, int bits);
 // Weight-streaming int8 products (qmv_a8_dense.hip): weight group 64, activation groups of 64 or 128.
 bool a8_dense_eligible(const AffineOp& op, const A8Operand& a, int bits);
-stark_qmm_status launch_a8_dense(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits,
+stark_qmm_status launch_a8_dense(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits, bool few,
                                  hipStream_t stream);
 uint32_t a8_gemm_class(const AffineOp& op, const A8Operand& a, int bits);
 stark_qmm_status launch_affine_a8_gemm_group(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits,

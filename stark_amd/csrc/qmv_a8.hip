@@ -18,6 +18,7 @@
 // meet in a wave reduction. Generic form (qmv_a8_generic): one thread per
 // output in the reference's order, for gathers and unaligned rows.
 #include "qmm_common.h"
+#include "dispatch_rules.h"
 
 namespace qmm {
 namespace {
@@ -520,32 +521,39 @@ uint32_t a8_gemm_class(const AffineOp& op, const A8Operand& a, int bits) {
            ((op.flags & FLAG_SIGNED) ? 2u : 0u) | (a.grouped ? 1u : 0u);
 }
 
-// Whether a launch goes to the weight-streaming kernel (qmv_a8_dense.hip): all
-// it can take, unless the GEMM's 128 x 128 tiles fill the chip more than twice
-// over, where its larger tiles are 5 to 13% faster (N 24576, K 4096: 384 rows,
-// 576 tiles 132 against 142 us, 2048 rows 534 against 557; N 4096, K 12288, 2048
-// rows, 512 tiles: 294 against 274; N 7424, K 1920: 1024 rows, 464 tiles 53.4
-// against 52.7, 1536 rows, 696 tiles 68 against 79).
-static bool a8_takes_dense(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits) {
+// Where a launch goes. Streaming (qmv_a8_dense.hip): all that it can take,
+// unless the GEMM's 128 x 128 tiles fill the chip more than twice over, where its
+// larger tiles are 5 to 13% faster (N 24576, K 4096: 384 rows, 576 tiles 132
+// against 142 us, 2048 rows 534 against 557; N 4096, K 12288, 2048 rows, 512
+// tiles: 294 against 274; N 7424, K 1920: 1024 rows, 464 tiles 53.4 against 52.7,
+// 1536 rows, 696 tiles 68 against 79), and but for a lone product of one or two
+// rows and few columns (a8_wave_per_row). few: products the GEMM does not take.
+struct A8Route {
+    bool dense, few;
+};
+static A8Route a8_route(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits) {
     uint64_t tiles = 0;
     bool gemm = true;
     for (uint32_t i = 0; i < count; ++i) {
-        if (!a8_dense_eligible(ops[i], as[i], bits)) return false;
-        gemm = gemm && (a8_gemm_eligible(ops[i], as[i], bits) || (uint64_t)ops[i].m * ops[i].k >= (1ull << 31));
+        if (!a8_dense_eligible(ops[i], as[i], bits)) return {false, false};
+        gemm = gemm && (a8_gemm_eligible(ops[i], as[i], bits) ||
+                        (ops[i].m > 16 && (uint64_t)ops[i].m * ops[i].k >= (1ull << 31)));
         tiles += a8_tiles(ops[i]);
     }
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return false;
-    return !gemm || tiles * 4 < (uint64_t)cus * 9;
+        return {false, false};
+    if (!gemm) return {count > 1 || !a8_wave_per_row(ops[0].m, ops[0].n, ops[0].k, bits, (uint32_t)cus), true};
+    return {tiles * 4 < (uint64_t)cus * 9, false};
 }
 
 stark_qmm_status launch_affine_a8_gemm_group(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits,
                                              hipStream_t stream) {
     if (count == 0) return STARK_QMM_OK;
     if (count > (uint32_t)kMaxBatchOps) return STARK_QMM_UNSUPPORTED;
-    if (a8_takes_dense(ops, as, count, bits)) return launch_a8_dense(ops, as, count, bits, stream);
+    const A8Route route = a8_route(ops, as, count, bits);
+    if (route.dense) return launch_a8_dense(ops, as, count, bits, route.few, stream);
     bool one = count == 1;
     for (uint32_t i = 0; i < count; ++i) one = one || !a8_gemm_eligible(ops[i], as[i], bits);
     if (one) {
@@ -583,7 +591,8 @@ stark_qmm_status launch_affine_a8_gemm_group(const AffineOp* ops, const A8Operan
 
 stark_qmm_status launch_affine_a8(const AffineOp& op, const A8Operand& a, int bits, hipStream_t stream) {
     if (op.m == 0 || op.n == 0) return STARK_QMM_OK;
-    if (a8_takes_dense(&op, &a, 1, bits)) return launch_a8_dense(&op, &a, 1, bits, stream);
+    const A8Route route = a8_route(&op, &a, 1, bits);
+    if (route.dense) return launch_a8_dense(&op, &a, 1, bits, route.few, stream);
     // a product too tall for one grid's 32-bit offsets: launches of whole rows
     // (the activation codes, their scales and d advanced per part)
     if (op.m > 16 && op.k > 0 && (uint64_t)op.m * op.k >= (1ull << 31)) {

@@ -37,6 +37,7 @@
 // (in the int8 MLP of 512 rows, between other kernels, the second one takes 108.7.)
 #include "qmm_common.h"
 #include "code_layout.h"
+#include "dispatch_rules.h"
 
 namespace qmm {
 namespace {
@@ -338,38 +339,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
 }
 
-// Shapes (16-row blocks, waves along K), two workgroups per CU each, and the
-// measured time of one pass of 128 KW values with the second workgroup of each
-// CU (full) and without (half), in us; a round also pays about 4 us of first
-// loads and last sums.
-struct Shape {
-    int mt, kw;
-    double full, half;
-};
-constexpr Shape kShapes[] = {{1, 8, 1.5, 1.0}, {2, 8, 2.3, 1.65}, {2, 4, 2.1, 1.25}, {2, 2, 2.0, 1.1},
-                             {4, 2, 3.1, 1.8}, {4, 1, 2.5, 1.65}};
-constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
-
-uint64_t shape_tiles(const Shape& s, const AffineOp& o) {
-    const uint32_t cols = 32 * (kWaves / s.kw), rows = 16 * s.mt;
-    return (uint64_t)((o.n + cols - 1) / cols) * ((o.m + rows - 1) / rows);
-}
-
-// Estimated time of the launch in a shape: whole rounds of two workgroups per CU, and the rest.
-double shape_cost(const Shape& s, const AffineOp* ops, uint32_t count, uint32_t cus) {
-    uint64_t tiles = 0;
-    double passes = 0;
-    for (uint32_t i = 0; i < count; ++i) {
-        const uint64_t t = shape_tiles(s, ops[i]);
-        tiles += t;
-        passes += (double)t * ((ops[i].k + 128 * s.kw - 1) / (128 * s.kw));
-    }
-    passes /= std::max<uint64_t>(tiles, 1);
-    const uint64_t rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
-    const double full = 4.0 + passes * s.full, half = 4.0 + passes * s.half;
-    return rounds * full + (rest > cus ? full : rest ? half : 0.0);
-}
-
 template <int MT, int KW>
 void launch_shape(const A8Batch& b, int bits, uint32_t tiles, hipStream_t stream) {
     const bool bf = b.op[0].w_dt == STARK_QMM_BF16;
@@ -390,33 +359,22 @@ bool a8_dense_eligible(const AffineOp& o, const A8Operand& a, int bits) {
            (((uintptr_t)o.scales | (uintptr_t)o.corr) & 1) == 0;
 }
 
-// ops: all a8_dense_eligible for `bits`, of one plane type.
-stark_qmm_status launch_a8_dense(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits,
+// ops: all a8_dense_eligible for `bits`, of one plane type. few: products that the GEMM does not take.
+stark_qmm_status launch_a8_dense(const AffineOp* ops, const A8Operand* as, uint32_t count, int bits, bool few,
                                  hipStream_t stream) {
     if (count == 0) return STARK_QMM_OK;
     if (count > (uint32_t)kMaxBatchOps) return STARK_QMM_UNSUPPORTED;
     int dev = 0, cus = 0;
     QMM_HIP_CHECK(hipGetDevice(&dev));
     QMM_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    uint32_t rows = 0;
-    for (uint32_t i = 0; i < count; ++i) rows = std::max(rows, ops[i].m);
-    // up to 16 rows the first shape, whose sums are the most exact ones
-    int best = 0;
-    double cost = 0;
-    for (int i = 0; i < (rows <= 16 ? 1 : kShapeCount); ++i) {
-        const double c = shape_cost(kShapes[i], ops, count, (uint32_t)std::max(cus, 1));
-        if (i == 0 || c < cost) {
-            best = i;
-            cost = c;
-        }
-    }
+    const int best = a8_shape(ops, count, few, (uint32_t)cus);
     A8Batch b{};
     uint64_t tiles = 0;
     for (uint32_t i = 0; i < count; ++i) {
         b.op[i] = ops[i];
         b.a[i] = as[i];
         b.op[i].block_begin = (uint32_t)tiles;
-        tiles += shape_tiles(kShapes[best], ops[i]);
+        tiles += a8_shape_tiles(kA8Shapes[best], ops[i]);
         if (tiles > 0x7fffffffu) return STARK_QMM_UNSUPPORTED;
     }
     b.count = count;

@@ -1,0 +1,55 @@
+"""The dispatch rules of stark_amd/csrc/dispatch_rules.h, compiled for the CPU,
+so that a test can say which kernel or shape its sizes get."""
+import ctypes as C
+import functools
+import os
+import subprocess
+import tempfile
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "stark_amd", "csrc")
+CUS = 256  # of an MI355X
+
+_WRAP = """
+#include "dispatch_rules.h"
+struct Op { uint32_t m, n, k; };
+extern "C" {
+int a8_wave_per_row(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t cus) {
+    return qmm::a8_wave_per_row(m, n, k, bits, cus);
+}
+int a8_shape(const Op* ops, uint32_t count, int few, uint32_t cus, int* mt, int* kw) {
+    const qmm::A8Shape& s = qmm::kA8Shapes[qmm::a8_shape(ops, count, few != 0, cus)];
+    *mt = s.mt;
+    *kw = s.kw;
+    return 0;
+}
+}
+"""
+
+
+class Op(C.Structure):
+    _fields_ = [("m", C.c_uint32), ("n", C.c_uint32), ("k", C.c_uint32)]
+
+
+@functools.lru_cache(None)
+def rules():
+    with tempfile.TemporaryDirectory() as d:
+        src, lib = os.path.join(d, "rules.cpp"), os.path.join(d, "rules.so")
+        with open(src, "w") as f:
+            f.write(_WRAP)
+        subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, src, "-o", lib], check=True)
+        return C.CDLL(lib)
+
+
+def ops(*sizes):
+    return (Op * len(sizes))(*[Op(*s) for s in sizes])
+
+
+def a8_wave_per_row(m, n, k, bits, cus=CUS):
+    return bool(rules().a8_wave_per_row(m, n, k, bits, cus))
+
+
+def a8_shape(sizes, few, cus=CUS):
+    """(16-row blocks, waves along K) of a launch of products (m, n, k)."""
+    mt, kw = C.c_int(), C.c_int()
+    rules().a8_shape(ops(*sizes), len(sizes), int(few), cus, C.byref(mt), C.byref(kw))
+    return mt.value, kw.value

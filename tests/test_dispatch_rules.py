@@ -1,0 +1,45 @@
+"""Which kernel or shape a size gets (CPU; the rules of csrc/dispatch_rules.h at
+the 256 CUs of an MI355X): the sizes of the GPU tests reach what they are there
+for, and at the measured sizes the rule takes the faster side."""
+import pytest
+
+from tests import dispatch as D
+from tests import test_gpu_a8_dense as A8
+
+
+def test_a8_shape_cases_reach_every_shape():
+    for m, n, k, _, shape in A8.SHAPES:
+        assert D.a8_shape([(m, n, k)], few=m <= 16) == shape, (m, n, k)
+        passes = -(-k // (128 * shape[1]))
+        assert passes >= 4 and k // 64 % 2 == 1
+    assert len({c[-1] for c in A8.SHAPES}) == 6
+
+
+def test_a8_few_rows_take_the_exact_shape():
+    for m in (1, 5, 16):
+        for n in (40, 16500, 200000):
+            assert D.a8_shape([(m, n, 4096)], few=True) == (1, 8)
+
+
+def test_a8_row_cases_are_on_both_sides():
+    for m, n, k, wave4, wave8 in A8.ROWS:
+        assert D.a8_wave_per_row(m, n, k, 4) == wave4 and D.a8_wave_per_row(m, n, k, 8) == wave8, (m, n, k)
+    for m in (1, 2):
+        for side in (3, 4):
+            assert {c[side] for c in A8.ROWS if c[0] == m} == {True, False}
+    assert not D.a8_wave_per_row(3, 64, 64, 4) and not D.a8_wave_per_row(3, 64, 64, 8)
+
+
+# bits, rows, n, k, us with a wave a row, us streaming (one MI355X, graph replays over weight copies)
+MEASURED = [(4, 1, 256, 8192, 7.24, 10.07), (4, 1, 512, 2048, 3.27, 4.27), (4, 1, 1024, 1024, 3.24, 3.59),
+            (4, 1, 2048, 8192, 9.11, 10.23), (4, 1, 2304, 4096, 6.40, 6.75), (4, 1, 2560, 2048, 4.83, 5.07),
+            (4, 1, 2560, 1024, 4.49, 4.33), (4, 1, 3584, 4096, 7.24, 6.85), (4, 1, 4608, 1024, 5.14, 4.47),
+            (4, 2, 1024, 4096, 6.29, 6.75), (4, 2, 1024, 8192, 8.98, 10.23), (8, 1, 1024, 1024, 3.48, 4.59),
+            (8, 1, 2560, 512, 3.71, 4.60), (8, 1, 3072, 1024, 4.62, 4.78), (8, 1, 1024, 2048, 4.59, 5.48),
+            (8, 1, 512, 4096, 6.53, 7.28), (8, 1, 4608, 1024, 5.18, 4.93), (8, 1, 1536, 2048, 5.80, 5.46),
+            (8, 1, 1024, 8192, 12.36, 11.53), (8, 2, 2048, 1024, 4.21, 4.80), (8, 2, 3072, 512, 4.28, 4.71)]
+
+
+@pytest.mark.parametrize("bits,m,n,k,wave,stream", MEASURED)
+def test_a8_row_rule_takes_the_faster_side(bits, m, n, k, wave, stream):
+    assert D.a8_wave_per_row(m, n, k, bits) == (wave < stream)

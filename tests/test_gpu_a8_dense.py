@@ -1,8 +1,10 @@
 """Int8-activation products on the weight-streaming kernel: every workgroup shape
-its rule can choose (rows of 1 to 16, to 32 and more; few and many columns),
-edges of its tiles (rows, 32 to 256 columns) and passes (odd group counts),
-planes of any alignment, both code layouts, activation groups of 64 and 128,
-corrections, codes and D-ops, against the oracle (bar of tests/tolerances.py)."""
+its rule can choose, over several passes and an odd last group (SHAPES; which
+shape a size gets is asserted on the CPU, test_dispatch_rules.py), both sides of
+the rule that leaves one or two rows of few columns to a wave a row (ROWS), edges
+of its tiles (rows, 32 to 256 columns) and passes, planes of any alignment, both
+code layouts, activation groups of 64 and 128, corrections, codes and D-ops,
+against the oracle (bar of tests/tolerances.py)."""
 import numpy as np
 import pytest
 import torch
@@ -50,6 +52,28 @@ def _run(Q, O, m, n, k, bits, ag, grouped, layout, correction=1, signed=False, w
                                       (150, 5000, 320, 64)])
 def test_shapes(qmm, oracle, bits, grouped, m, n, k, ag):
     _run(qmm, oracle, m, n, k, bits, ag, grouped, layout=(m + n) % 2)
+
+
+# (m, n, k, activation group) and the shape (16-row blocks, waves along K): passes of 128 values a wave, at least 4 and an odd group
+SHAPES = [(17, 40, 4160, 64, (1, 8)), (19, 8310, 4672, 64, (2, 8)), (17, 8310, 2112, 64, (2, 4)),
+          (33, 8310, 1088, 64, (2, 2)), (50, 16510, 1088, 64, (4, 2)), (35, 33010, 576, 64, (4, 1))]
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k,ag,shape", SHAPES)
+def test_each_shape(qmm, oracle, bits, m, n, k, ag, shape):
+    _run(qmm, oracle, m, n, k, bits, ag, grouped=bits == 8, layout=(shape[0] + shape[1]) % 2)
+
+
+# one and two rows (m, n, k), and whether 4-bit and 8-bit ones take a wave a row
+ROWS = [(1, 700, 2112, True, True), (1, 3200, 2112, False, False), (1, 2304, 1024, True, True), (1, 600, 576, False, True),
+        (2, 500, 2112, True, False), (2, 1030, 2112, False, False), (2, 500, 832, False, True)]
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k,wave4,wave8", ROWS)
+def test_one_and_two_rows(qmm, oracle, bits, m, n, k, wave4, wave8):
+    _run(qmm, oracle, m, n, k, bits, 64, grouped=n % 3 == 0, layout=(m + k // 64) % 2)
 
 
 @pytest.mark.parametrize("bits", [4, 8])
