@@ -220,7 +220,7 @@ stark_qmm_status encode_product(stark_qmm_kernel* kr, const stark_qmm_args* args
     return launch_affine_generic(op, bits, stream);
 }
 
-// The int8-activation GEMM operands of args when the product takes that grid
+// The int8-activation operands of args when the product takes a grid shared with others
 // with the same validation as encode_product (else false: the entry then
 // goes through stark_qmm_encode, which reports any error).
 bool a8_gemm_entry(const stark_qmm_kernel* kr, const stark_qmm_args* a, AffineOp* op, A8Operand* q, int* bits) {
@@ -237,7 +237,9 @@ bool a8_gemm_entry(const stark_qmm_kernel* kr, const stark_qmm_args* a, AffineOp
     if (!a->d || (a->k && (!a->a || !a->a_scales))) return false;
     *q = A8Operand{(const int8_t*)a->a, a->a_scales, a->a_scale_group_size,
                    a->a_code_layout == STARK_QMM_CODES_GROUPED_BY_NIBBLE ? 1u : 0u};
-    return a8_gemm_eligible(*op, *q, *bits) || a8_dense_eligible(*op, *q, *bits);
+    // (a product too tall for one GEMM grid is cut into rows by stark_qmm_encode)
+    return a8_gemm_eligible(*op, *q, *bits) ||
+           (a8_dense_eligible(*op, *q, *bits) && (a->m <= 16 || (uint64_t)a->m * a->k < (1ull << 31)));
 }
 
 }  // namespace
@@ -268,9 +270,10 @@ stark_qmm_status stark_qmm_encode_many(stark_qmm_kernel* kr, const stark_qmm_arg
     // prefill-sized products by (bits, signed codes, biases, bf16 planes): one grid each
     std::vector<AffineOp> gemm[2][2][2][2];
     std::vector<AffineOp> streamed[2][2];  // by bits, plane type
-    // int8-activation prefill products by grid class
-    std::vector<AffineOp> a8_ops[16];
-    std::vector<A8Operand> a8_as[16];
+    // int8-activation products by grid class; those that the GEMM does not take
+    // (up to 16 rows) apart, whose launch has a rule of its own
+    std::vector<AffineOp> a8_ops[32];
+    std::vector<A8Operand> a8_as[32];
     std::vector<size_t> rest;
     const size_t xsz = kr->x_dt == STARK_QMM_F32 ? 4 : 2;
     for (uint32_t i = 0; i < count; ++i) {
@@ -281,7 +284,7 @@ stark_qmm_status stark_qmm_encode_many(stark_qmm_kernel* kr, const stark_qmm_arg
             A8Operand q;
             int bits;
             if (a8_gemm_entry(kr, a, &op, &q, &bits)) {
-                const uint32_t c = a8_gemm_class(op, q, bits);
+                const uint32_t c = a8_gemm_class(op, q, bits) | (a8_gemm_eligible(op, q, bits) ? 0u : 16u);
                 a8_ops[c].push_back(op);
                 a8_as[c].push_back(q);
                 continue;
@@ -349,7 +352,7 @@ stark_qmm_status stark_qmm_encode_many(stark_qmm_kernel* kr, const stark_qmm_arg
                         const stark_qmm_status st = launch_affine_gemm_group(v.data() + s, n, b8 ? 8 : 4, stream);
                         if (st != STARK_QMM_OK) return st;
                     }
-    for (uint32_t c = 0; c < 16; ++c)
+    for (uint32_t c = 0; c < 32; ++c)
         for (size_t s = 0; s < a8_ops[c].size(); s += kMaxBatchOps) {
             const uint32_t n = (uint32_t)std::min<size_t>(kMaxBatchOps, a8_ops[c].size() - s);
             const stark_qmm_status st =

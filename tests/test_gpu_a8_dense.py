@@ -114,3 +114,28 @@ def test_few_rows_round_as_one_row_a_wave(qmm, bits, k):
     w = codes.double().view(n, -1, 64) * s.double().unsqueeze(2) + b.double().unsqueeze(2)
     want = (q.double().view(m, -1, 64) * sa.double().unsqueeze(2)).view(m, k) @ w.view(n, k).t().contiguous()
     assert ((d.double() - want).norm() / want.norm()).item() < 1.05e-7
+
+
+def test_rows_in_one_call_do_not_meet(qmm, oracle):
+    """Few and many rows in one call: each as alone, bit for bit (the few ones
+    keep their own shape, and neither holds the other on a kernel that it would
+    not take)."""
+    rng = np.random.default_rng(11)
+    kern = qmm.MatmulKernel(H.BF16, H.BF16, H.F32)
+    args, outs = [], []
+    for m, n, k in ((5, 300, 1088), (300, 2200, 1088)):
+        w = H.affine_weights(oracle, rng, n, k, 4, 64, 1, 1, H.BF16)
+        a = qmm.Int8SymmetricA(values=H.to_dev(rng.integers(-127, 128, (m, k)).astype(np.int8)),
+                               scales=H.to_dev(rng.uniform(0.01, 0.1, (m, k // 64)).astype(np.float32)),
+                               scale_group_size=64, code_layout=qmm.SEQUENTIAL)
+        b = qmm.QuantizedB(codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), params=qmm.QuantParams(1, n, k // 64),
+                           correction_data=H.to_dev(w["corr"]))
+        for _ in range(2):
+            outs.append(torch.zeros(m * n, dtype=torch.float32, device="cuda"))
+            args.append(qmm.MatmulArguments(a=a, b=b, d=outs[-1], m=m, n=n, k=k))
+    kern.encode_many(args[0::2])
+    for a in args[1::2]:
+        kern.encode(a)
+    torch.cuda.synchronize()
+    for a, b in zip(outs[0::2], outs[1::2]):
+        assert torch.equal(a, b)
