@@ -79,4 +79,72 @@ inline bool a8_wave_per_row(uint32_t m, uint32_t n, uint32_t k, int bits, uint32
     return weights <= (k <= 1024 ? 14 : 8) * unit;
 }
 
+// ---- Products of up to 16 rows, group 64: qmv_dense (32-column tiles, two
+// workgroups per CU, 1024 values a pass) or qmv_mfma (16-column tiles, three per
+// CU, in 64-column groups dealt to the XCDs). Over the products of one launch.
+
+// Columns and 32-column tiles of a launch, and the depth that most of its weights have.
+struct LaunchSize {
+    uint64_t columns = 0, tiles = 0;
+    uint32_t k = 0;
+    bool mixed = false;  // products of different depths
+    bool even = true;    // qmv_mfma's groups come out even over the eight XCDs: a multiple of 512 columns in all
+};
+template <class Op>
+LaunchSize launch_size(const Op* ops, uint32_t count) {
+    LaunchSize z;
+    double most = -1;
+    for (uint32_t i = 0; i < count; ++i) {
+        z.columns += ops[i].n;
+        z.tiles += (ops[i].n + 31) / 32;
+        z.mixed = z.mixed || ops[i].k != ops[0].k;
+        z.even = z.even && ops[i].n % 64 == 0;
+        double weights = 0;
+        for (uint32_t j = 0; j < count; ++j) weights += ops[j].k == ops[i].k ? (double)ops[j].n * ops[j].k : 0.0;
+        if (weights > most) {
+            most = weights;
+            z.k = ops[i].k;
+        }
+    }
+    z.even = z.even && z.columns % 512 == 0;
+    return z;
+}
+
+// One or two rows.
+// idle: 4-bit, whose qmv_mfma passes of 2048 values run past K: all are dense, in
+// one launch (hidden 3072 / 8192, seven products: 19.9 us with the 8192-deep one
+// on its own kernel, 15.1 together, 16.3 on qmv_mfma). One depth: from 15% of the
+// weights walked for nothing on (two of 6912 x 2560, 38%: 9.1 against 7.5 us;
+// 9984 x 3328, 19%: 11.7 and 11.7). Products of several depths, whose tiles the
+// lists of qmv_mfma even out better: from 19.5% (3072 / 8192, 20%: above;
+// 1536 / 6144, 19%: 8.4 against 9.4; 3328 / 9984, 15%: 17.9 against 20.2), and not
+// when its columns come out even and the dense tiles are few (1024 / 2048 to
+// 4096, 42 to 46%: 4.7 to 5.8 against 5.4 to 6.6).
+// drag: products beside one whose planes qmv_mfma cannot read join it: a second
+// launch costs 3 to 6 us (8-bit 2560 / 6912: 23.3 against 26.5; 4-bit 2048 / 5568:
+// 9.3 against 15.2), the dense kernel about 10% of their time, which is more from
+// 160 MB on.
+struct FewRowsRule {
+    bool idle, drag;
+};
+template <class Op, class Readable>
+FewRowsRule few_rows_rule(const Op* ops, uint32_t count, int bits, uint32_t cus, Readable readable) {
+    double walked = 0, used = 0, others = 0;
+    bool unreadable = false, mixed = false;
+    for (uint32_t i = 0; i < count; ++i) {
+        const Op& o = ops[i];
+        mixed = mixed || o.k != ops[0].k;
+        walked += (double)o.n * ((o.k + 2047) / 2048 * 2048);
+        used += (double)o.n * o.k;
+        if (!readable(o)) unreadable = true;
+        else others += (double)o.n * o.k * bits / 8;
+    }
+    bool idle = bits == 4 && used < (mixed ? 0.805 : 0.85) * walked;
+    if (idle && mixed) {
+        const LaunchSize z = launch_size(ops, count);
+        idle = !(z.even && 2 * z.tiles <= 3 * (uint64_t)cus);
+    }
+    return {idle, unreadable && others < 160e6};
+}
+
 }  // namespace qmm

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/stark_qmm.h"
+#include "dispatch_rules.h"
 
 #define QMM_DEVICE __device__ __forceinline__
 
@@ -251,8 +252,8 @@ bool dense_eligible(const AffineOp& op, int bits);
 // Which products of one call it takes.
 struct DenseRule {
     int bits;
-    bool two_rows;  // products of one or two rows
-    bool many_rows;  // 4-bit products of more than eight
+    FewRowsRule few_rows;  // products of one or two rows
+    bool many_rows;        // 4-bit products of more than eight
     DenseRule(const AffineOp* ops, uint32_t count, int bits);
     bool takes(const AffineOp& op) const;
 };

@@ -18,7 +18,6 @@
 // meet in a wave reduction. Generic form (qmv_a8_generic): one thread per
 // output in the reference's order, for gathers and unaligned rows.
 #include "qmm_common.h"
-#include "dispatch_rules.h"
 
 namespace qmm {
 namespace {

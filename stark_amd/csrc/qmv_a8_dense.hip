@@ -37,7 +37,6 @@
 // (in the int8 MLP of 512 rows, between other kernels, the second one takes 108.7.)
 #include "qmm_common.h"
 #include "code_layout.h"
-#include "dispatch_rules.h"
 
 namespace qmm {
 namespace {

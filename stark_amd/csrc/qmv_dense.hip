@@ -326,34 +326,43 @@ bool dense_eligible(const AffineOp& o, int bits) {
 //    faster unless qmv_small_m gets long runs (small_m_long);
 //  - 8-bit: faster from 5 rows (hidden 4096 / 11008: 199 -> 178 at 6 rows, 295 ->
 //    214 at 16; 155 -> 168 at 3);
-//  - 4-bit, one or two rows: qmv_mfma walks K in passes of 2048 values, and the
-//    part of its last pass past K is idle: dense wins while that idle share of
-//    the weights is above 15% (hidden 2560 / 6912, 32%: 60 -> 56; 3072 / 8192,
-//    19%: 68 -> 62, 73 -> 64; 3584 / 9728, 11%: 77 -> 79, 88 -> 85; 2048 / 6144,
-//    none: 39 -> 44, 40 -> 45); 8-bit ones stay (1024-value passes; hidden 4096 /
-//    11008: 147 -> 161) and so does qmv_stream (K % 4096 == 0: 85 -> 95).
-DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b) : bits(b), two_rows(false), many_rows(true) {
-    double bytes = 0, used = 0;
-    std::vector<AffineOp> many;
+//  - one or two rows: few_rows_rule (4-bit passes with an idle share: hidden 2560
+//    / 6912, 32%: 60 -> 56; 3584 / 9728, 11%: 77 -> 79, 88 -> 85; 2048 / 6144,
+//    none: 39 -> 44, 40 -> 45; 8-bit, 1024-value passes, hidden 4096 / 11008:
+//    147 -> 161; qmv_stream, K % 4096 == 0: 85 -> 95).
+DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
+    : bits(b), few_rows{false, false}, many_rows(true) {
+    const auto readable = [&](const AffineOp& o) { return mfma_eligible(o, bits); };
+    const auto cus = [] {
+        int dev = 0, n = 0;
+        return hipGetDevice(&dev) == hipSuccess &&
+                       hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess
+                   ? (uint32_t)n
+                   : 256u;
+    };
+    if (count == 1 && ops[0].m <= 2) {  // the call that is all launch: no copies, nothing asked of the device
+        if (dense_eligible(ops[0], bits)) few_rows = few_rows_rule(ops, 1, bits, 0u, readable);
+        return;
+    }
+    std::vector<AffineOp> few, many;
     for (uint32_t i = 0; i < count; ++i) {
         const AffineOp& o = ops[i];
         if (!dense_eligible(o, bits)) continue;
-        if (o.m > 8) many.push_back(o);
-        if (o.m > 2) continue;
-        if (!mfma_eligible(o, bits)) two_rows = true;
-        const uint32_t whole = (o.k + 2047) / 2048 * 2048;
-        bytes += (double)o.n * whole;
-        used += (double)o.n * o.k;
+        if (o.m <= 2) {
+            few.push_back(o);
+        } else if (o.m > 8) {
+            if (bits == 4) many.push_back(o);
+        }
     }
-    if (bits == 4 && used < 0.85 * bytes) two_rows = true;
-    if (bits == 4 && !many.empty() && small_m_eligible(many.data(), (uint32_t)many.size()))
+    if (!few.empty()) few_rows = few_rows_rule(few.data(), (uint32_t)few.size(), bits, cus(), readable);
+    if (!many.empty() && small_m_eligible(many.data(), (uint32_t)many.size()))
         many_rows = !small_m_long(many.data(), (uint32_t)many.size());
 }
 
 bool DenseRule::takes(const AffineOp& o) const {
     if (!dense_eligible(o, bits)) return false;
     if (!mfma_eligible(o, bits)) return true;
-    if (o.m <= 2) return two_rows && !(bits == 4 && o.m == 1 && o.k % 4096 == 0);
+    if (o.m <= 2) return few_rows.idle || few_rows.drag;
     if (bits == 8) return o.m > 4;
     return o.m <= 8 || many_rows || !small_m_eligible(&o, 1);
 }

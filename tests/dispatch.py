@@ -22,6 +22,11 @@ int a8_shape(const Op* ops, uint32_t count, int few, uint32_t cus, int* mt, int*
     *kw = s.kw;
     return 0;
 }
+int few_rows(const Op* ops, const int* readable, uint32_t count, int bits, uint32_t cus) {
+    const auto read = [&](const Op& o) { return readable[&o - ops] != 0; };
+    const qmm::FewRowsRule r = qmm::few_rows_rule(ops, count, bits, cus, read);
+    return (r.idle ? 1 : 0) | (r.drag ? 2 : 0);
+}
 }
 """
 
@@ -53,3 +58,10 @@ def a8_shape(sizes, few, cus=CUS):
     mt, kw = C.c_int(), C.c_int()
     rules().a8_shape(ops(*sizes), len(sizes), int(few), cus, C.byref(mt), C.byref(kw))
     return mt.value, kw.value
+
+
+def few_rows(sizes, bits, readable=None, cus=CUS):
+    """(idle, drag) of a launch's products of one or two rows; readable: those whose planes qmv_mfma can read."""
+    flags = (C.c_int * len(sizes))(*([1] * len(sizes) if readable is None else [int(r) for r in readable]))
+    r = rules().few_rows(ops(*sizes), flags, len(sizes), bits, cus)
+    return bool(r & 1), bool(r & 2)

@@ -43,3 +43,36 @@ MEASURED = [(4, 1, 256, 8192, 7.24, 10.07), (4, 1, 512, 2048, 3.27, 4.27), (4, 1
 @pytest.mark.parametrize("bits,m,n,k,wave,stream", MEASURED)
 def test_a8_row_rule_takes_the_faster_side(bits, m, n, k, wave, stream):
     assert D.a8_wave_per_row(m, n, k, bits) == (wave < stream)
+
+
+def _layer(m, hidden, inter):
+    kv = hidden // 4 // 64 * 64
+    return [(m, hidden, hidden), (m, kv, hidden), (m, kv, hidden), (m, hidden, hidden), (m, inter, hidden),
+            (m, inter, hidden), (m, hidden, inter)]
+
+
+def _pair(m, hidden, inter):
+    return [(m, inter, hidden)] * 2
+
+
+# 4-bit, one row: products of a call, us on qmv_mfma, us dense (differences of 2% and more)
+MEASURED_IDLE = [(_layer(1, 3072, 8192), 16.4, 15.4), (_layer(1, 2560, 6912), 14.6, 14.0), (_layer(1, 1536, 4096), 7.65, 7.08),
+                 (_layer(1, 1280, 3584), 7.47, 6.81), (_layer(1, 2816, 8448), 16.5, 15.7), (_layer(1, 512, 1536), 6.69, 3.82),
+                 (_layer(1, 1024, 2048), 4.69, 5.36), (_layer(1, 1024, 4096), 5.80, 6.58), (_layer(1, 1536, 6144), 8.43, 9.37),
+                 (_layer(1, 3328, 9984), 17.9, 20.2), (_pair(1, 1024, 3072), 4.65, 3.38), (_pair(1, 2560, 6912), 9.06, 7.45),
+                 (_pair(1, 3072, 8192), 9.82, 7.97), (_layer(1, 2048, 6144), 9.7, 11.0), ([(1, 3072, 8192)], 1.0, 1.1)]
+
+
+@pytest.mark.parametrize("sizes,mfma,dense", MEASURED_IDLE)
+def test_idle_rule_takes_the_faster_side(sizes, mfma, dense):
+    assert D.few_rows(sizes, 4)[0] == (dense < mfma)
+    assert D.few_rows(sizes, 8) == (False, False)
+
+
+def test_unreadable_products_drag_what_a_second_launch_costs_more_for():
+    for bits in (4, 8):
+        layer = _layer(1, 2560, 6912)
+        assert D.few_rows(layer, bits, readable=[True] * 6 + [False])[1]
+        # a small one beside 600 MB stays alone
+        big = [(1, 100, 4096), (1, 151936 * 8 // bits, 4096)]
+        assert not D.few_rows(big, bits, readable=[False, True])[1]

@@ -10,6 +10,7 @@ import torch
 
 from tests import helpers as H
 from tests import test_gpu_affine as A
+from tests.tolerances import check
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +28,38 @@ def test_dense_shapes(qmm, oracle, bits, layout, m, n, k):
 def test_dense_corrections(qmm, oracle, correction, signed, w_dt, bits, m):
     A.run_case(qmm, oracle, n=72, k=1216, m=m, bits=bits, gs=64, layout=0, correction=correction, signed=signed, w_dt=w_dt,
            seed=m)
+
+
+@pytest.mark.parametrize("m", [1, 2])
+def test_few_rows_in_one_launch(qmm, oracle, m):
+    """A launch whose shorter products leave qmv_mfma's passes idle: all of them
+    dense, the 4096-deep one (another kernel's when alone) included; and a
+    product with unreadable planes beside readable ones, dragged and (past 160
+    MB of others) not: each as the oracle has it."""
+    rng = np.random.default_rng(m)
+    kern = qmm.MatmulKernel(H.BF16, H.BF16, H.F32)
+    for sizes in (((64, 1088), (48, 1088), (32, 4096)), ((33, 704), (64, 1024), (64, 4096)), ((33, 704), (81920, 4096))):
+        args, cases = [], []
+        for n, k in sizes:
+            w = H.affine_weights(oracle, rng, min(n, 64), k, 4, 64, 0, 1, H.BF16)
+            reps = -(-n // 64)  # a wide product repeats its rows
+            x = H.activations(oracle, rng, m, k, H.BF16)
+            codes, s, b = (H.to_dev(np.tile(w[key].reshape(min(n, 64), -1), (reps, 1)).ravel()) for key in ("codes", "scales", "corr"))
+            d = torch.zeros(m * n, dtype=torch.float32, device="cuda")
+            args.append(qmm.MatmulArguments(a=H.to_dev(x), m=m, n=n, k=k, d=d,
+                                            b=qmm.QuantizedB(codes=codes, scales=s, correction_data=b,
+                                                             params=qmm.QuantParams(0, n, k // 64))))
+            cases.append((w, x, min(n, 64), k, n, d))
+        kern.encode_many(args)
+        torch.cuda.synchronize()
+        for w, x, rows, k, n, d in cases:
+            st, want = oracle.matmul(a=x, m=m, n=rows, k=k, codes=w["codes"], scales=w["scales"], correction_data=w["corr"],
+                                     layout=0, bits=4, group_size=64, output_dt=H.F32, threads=8)
+            assert st == 0
+            mag = H.dequant_magnitude(oracle, w["codes"], w["scales"], w["corr"], rows, k, 4, 64, 0, 1, H.BF16, x, H.BF16, m)
+            got = d.cpu().numpy().reshape(m, n)
+            for r in (0, n - rows):
+                check(got[:, r:r + rows].ravel(), want, mag=mag, label=f"m{m} n{n} k{k} at {r}")
 
 
 @pytest.mark.parametrize("bits", [4, 8])
