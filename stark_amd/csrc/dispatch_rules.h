@@ -147,4 +147,29 @@ FewRowsRule few_rows_rule(const Op* ops, uint32_t count, int bits, uint32_t cus,
     return {idle, unreadable && others < 160e6};
 }
 
+// Whether qmv_mfma takes a launch's 8-bit products of 5 to 8 rows, all of which
+// it can read. Its columns have to come out even (else some workgroup has two
+// tiles where others have one: N 6912, K 4096 21.1 us against 10.1), and it is then
+// the faster one where the dense tiles come out badly: between one and 1.5 a CU
+// (N 12288, eight rows, K 1024 5.8 against 7.1, 2560 1.16 times, 4096 16.2 against
+// 16.9, 12288 39.8 against 45.1; at two passes, K 1025 to 2048, alike), and where
+// K is an odd number of passes, one above all (K 1024: N 4096 4.2 against 4.7,
+// 24576 9.6 against 10.9, 8192 and 16384 alike, two of 4096 5.1 against 5.5; N
+// 27648: K 3072 25.4 against 27.1, 5120 39.1 against 43.0, 4096 32.6 against 30.3,
+// 7168 52.6 against 54.4). Of several depths and many tiles also without even
+// columns (seven products, hidden 2304 / 6912 22.9 against 24.6, 2560 / 6912 25.1
+// against 26.1, 5120 / 13824 72.2 against 75.2; 4096 / 11008 47.0 against 44.5).
+template <class Op>
+bool w8_rows5_mfma(const Op* ops, uint32_t count, uint32_t cus) {
+    if (count == 0) return false;
+    const LaunchSize z = launch_size(ops, count);
+    const uint32_t passes = (z.k + 1023) / 1024;
+    const bool many = z.tiles > 2 * (uint64_t)cus;
+    if (z.mixed && many) return passes % 2 == 1 && passes <= 5;
+    if (!z.even) return false;
+    if (z.tiles > cus && 2 * z.tiles <= 3 * (uint64_t)cus) return passes != 2;
+    if (passes == 1) return many || (16 * z.tiles >= 3 * (uint64_t)cus && (count > 1 ? 1 : 2) * z.tiles <= cus);
+    return many && z.k % 2048 == 1024 && passes <= 5;
+}
+
 }  // namespace qmm

@@ -254,6 +254,7 @@ struct DenseRule {
     int bits;
     FewRowsRule few_rows;  // products of one or two rows
     bool many_rows;        // 4-bit products of more than eight
+    bool mid_rows;         // 8-bit products of five to eight
     DenseRule(const AffineOp* ops, uint32_t count, int bits);
     bool takes(const AffineOp& op) const;
 };

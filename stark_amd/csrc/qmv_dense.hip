@@ -324,14 +324,15 @@ bool dense_eligible(const AffineOp& o, int bits) {
 //  - 4-bit, 3 to 8 rows: always faster (hidden 4096 / 12288: 123 -> 101, 126 ->
 //    120, 135 -> 128 at 3, 5, 8 rows; 2048 / 6144: 70 -> 49 at 5); 9 to 16 rows:
 //    faster unless qmv_small_m gets long runs (small_m_long);
-//  - 8-bit: faster from 5 rows (hidden 4096 / 11008: 199 -> 178 at 6 rows, 295 ->
-//    214 at 16; 155 -> 168 at 3);
+//  - 8-bit: faster from 9 rows, and from 5 unless the tiles come out badly
+//    (w8_rows5_mfma; hidden 4096 / 11008: 199 -> 178 at 6 rows, 295 -> 214 at 16;
+//    155 -> 168 at 3);
 //  - one or two rows: few_rows_rule (4-bit passes with an idle share: hidden 2560
 //    / 6912, 32%: 60 -> 56; 3584 / 9728, 11%: 77 -> 79, 88 -> 85; 2048 / 6144,
 //    none: 39 -> 44, 40 -> 45; 8-bit, 1024-value passes, hidden 4096 / 11008:
 //    147 -> 161; qmv_stream, K % 4096 == 0: 85 -> 95).
 DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
-    : bits(b), few_rows{false, false}, many_rows(true) {
+    : bits(b), few_rows{false, false}, many_rows(true), mid_rows(true) {
     const auto readable = [&](const AffineOp& o) { return mfma_eligible(o, bits); };
     const auto cus = [] {
         int dev = 0, n = 0;
@@ -344,7 +345,8 @@ DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
         if (dense_eligible(ops[0], bits)) few_rows = few_rows_rule(ops, 1, bits, 0u, readable);
         return;
     }
-    std::vector<AffineOp> few, many;
+    std::vector<AffineOp> few, mid, many;
+    bool mid_readable = true;
     for (uint32_t i = 0; i < count; ++i) {
         const AffineOp& o = ops[i];
         if (!dense_eligible(o, bits)) continue;
@@ -352,18 +354,22 @@ DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
             few.push_back(o);
         } else if (o.m > 8) {
             if (bits == 4) many.push_back(o);
+        } else if (o.m > 4 && bits == 8) {
+            mid.push_back(o);
+            mid_readable = mid_readable && readable(o);
         }
     }
     if (!few.empty()) few_rows = few_rows_rule(few.data(), (uint32_t)few.size(), bits, cus(), readable);
     if (!many.empty() && small_m_eligible(many.data(), (uint32_t)many.size()))
         many_rows = !small_m_long(many.data(), (uint32_t)many.size());
+    if (!mid.empty() && mid_readable) mid_rows = !w8_rows5_mfma(mid.data(), (uint32_t)mid.size(), cus());
 }
 
 bool DenseRule::takes(const AffineOp& o) const {
     if (!dense_eligible(o, bits)) return false;
     if (!mfma_eligible(o, bits)) return true;
     if (o.m <= 2) return few_rows.idle || few_rows.drag;
-    if (bits == 8) return o.m > 4;
+    if (bits == 8) return o.m > 8 || (o.m > 4 && mid_rows);
     return o.m <= 8 || many_rows || !small_m_eligible(&o, 1);
 }
 

@@ -808,8 +808,8 @@ stark_qmm_status launch_gs(const AffineOp* o, uint32_t n, hipStream_t st) {
         if constexpr (MP * MB == 16 && BITS == 4) {  // M = 9 .. 16
             if (small_m_eligible(o, n)) return launch_small_m(o, n, sg, st);
         }
-        // 4-bit products of 3 rows and 8-bit ones of 5 rows and more are qmv_dense's (DenseRule)
-        if constexpr (MP > (BITS == 4 ? 2 : 4)) return STARK_QMM_UNSUPPORTED;
+        // 4-bit products of 3 rows and 8-bit ones of 9 rows and more are qmv_dense's (DenseRule)
+        if constexpr (BITS == 4 ? MP > 2 : MP * MB > 8) return STARK_QMM_UNSUPPORTED;
         else return sg ? launch_one<MP, MB, 64, BITS, true>(o, n, st) : launch_one<MP, MB, 64, BITS, false>(o, n, st);
     default:
         return sg ? launch_one<MP, MB, 128, BITS, true>(o, n, st) : launch_one<MP, MB, 128, BITS, false>(o, n, st);

@@ -27,6 +27,7 @@ int few_rows(const Op* ops, const int* readable, uint32_t count, int bits, uint3
     const qmm::FewRowsRule r = qmm::few_rows_rule(ops, count, bits, cus, read);
     return (r.idle ? 1 : 0) | (r.drag ? 2 : 0);
 }
+int w8_rows5_mfma(const Op* ops, uint32_t count, uint32_t cus) { return qmm::w8_rows5_mfma(ops, count, cus); }
 }
 """
 
@@ -65,3 +66,7 @@ def few_rows(sizes, bits, readable=None, cus=CUS):
     flags = (C.c_int * len(sizes))(*([1] * len(sizes) if readable is None else [int(r) for r in readable]))
     r = rules().few_rows(ops(*sizes), flags, len(sizes), bits, cus)
     return bool(r & 1), bool(r & 2)
+
+
+def w8_rows5_mfma(sizes, cus=CUS):
+    return bool(rules().w8_rows5_mfma(ops(*sizes), len(sizes), cus))

@@ -5,6 +5,7 @@ import pytest
 
 from tests import dispatch as D
 from tests import test_gpu_a8_dense as A8
+from tests import test_gpu_affine_dense as AD
 
 
 def test_a8_shape_cases_reach_every_shape():
@@ -76,3 +77,24 @@ def test_unreadable_products_drag_what_a_second_launch_costs_more_for():
         # a small one beside 600 MB stays alone
         big = [(1, 100, 4096), (1, 151936 * 8 // bits, 4096)]
         assert not D.few_rows(big, bits, readable=[False, True])[1]
+
+
+# 8-bit, eight rows: products of a call, us on qmv_mfma, us dense
+MEASURED_W8 = [([(8, 12288, 4096)], 16.2, 16.9), ([(8, 12288, 1024)], 5.83, 7.06), ([(8, 12288, 12288)], 39.8, 45.1),
+               ([(8, 24576, 1024)], 9.61, 10.93), ([(8, 4096, 1024)], 4.22, 4.70), ([(8, 4096, 4096)], 10.9, 9.2),
+               ([(8, 6912, 4096)], 21.1, 10.1), ([(8, 6912, 1024)], 7.1, 4.95), ([(8, 14336, 1024)], 7.95, 7.29),
+               ([(8, 24576, 2048)], 16.7, 13.4), ([(8, 27648, 5120)], 39.1, 43.0), ([(8, 27648, 4096)], 32.6, 30.3),
+               ([(8, 11008, 4096)], 1.0, 0.76), (_pair(8, 1024, 4096), 5.05, 5.45), (_pair(8, 1024, 2816), 4.84, 5.23),
+               (_layer(8, 2304, 6912), 22.9, 24.6), (_layer(8, 2560, 6912), 25.1, 26.1), (_layer(8, 5120, 13824), 72.2, 75.2),
+               (_layer(8, 4096, 11008), 47.0, 44.5)]
+
+
+@pytest.mark.parametrize("sizes,mfma,dense", MEASURED_W8)
+def test_w8_rule_takes_the_faster_side(sizes, mfma, dense):
+    assert D.w8_rows5_mfma(sizes) == (mfma < dense)
+
+
+def test_w8_cases_reach_both_kernels():
+    for m, n, k, mfma in AD.W8_ROWS:
+        assert 5 <= m <= 8 and D.w8_rows5_mfma([(m, n, k)]) == mfma, (m, n, k)
+    assert {c[-1] for c in AD.W8_ROWS} == {True, False}

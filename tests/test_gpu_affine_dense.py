@@ -30,6 +30,17 @@ def test_dense_corrections(qmm, oracle, correction, signed, w_dt, bits, m):
            seed=m)
 
 
+# 8-bit products of five to eight rows (m, n, k), and whether the rule leaves them to qmv_mfma
+W8_ROWS = [(5, 1536, 448, True), (6, 2048, 1024, True), (8, 8704, 2112, True), (7, 1536, 1088, False), (8, 8192, 2112, False)]
+
+
+@pytest.mark.parametrize("m,n,k,mfma", W8_ROWS)
+def test_w8_five_to_eight_rows(qmm, oracle, m, n, k, mfma):
+    A.run_case(qmm, oracle, m=m, n=n, k=k, bits=8, gs=64, layout=1, seed=n + k + m)
+    A.run_case(qmm, oracle, m=m, n=n, k=k, bits=8, gs=64, layout=1, correction=0, signed=True, w_dt=H.F16, accumulate=True,
+               with_bias=True, seed=m)
+
+
 @pytest.mark.parametrize("m", [1, 2])
 def test_few_rows_in_one_launch(qmm, oracle, m):
     """A launch whose shorter products leave qmv_mfma's passes idle: all of them
