@@ -147,6 +147,19 @@ FewRowsRule few_rows_rule(const Op* ops, uint32_t count, int bits, uint32_t cus,
     return {idle, unreadable && others < 160e6};
 }
 
+// Whether a launch of 4-bit products of 9 to 16 rows, all of which it can take,
+// stays with qmv_small_m: what that saves is the activation stage of each 32
+// columns, through its runs, and those need many passes (32 columns x 1024
+// values) for each of its two resident workgroups a CU (16 rows: 11.5 passes
+// each on the seven products of 4096 / 12288, 154 us for four layers against
+// 169; 5.9 at 3072 / 8192, 109 against 106; 2.2 at 2048 / 6144, 87 against 62).
+template <class Op>
+bool small_m_long(const Op* ops, uint32_t count, uint32_t cus) {
+    uint64_t units = 0;
+    for (uint32_t i = 0; i < count; ++i) units += (uint64_t)((ops[i].n + 31) / 32) * (ops[i].k / 1024);
+    return units >= 8 * 2 * (uint64_t)cus;
+}
+
 // Whether qmv_mfma takes a launch's 8-bit products of 5 to 8 rows, all of which
 // it can read. Its columns have to come out even (else some workgroup has two
 // tiles where others have one: N 6912, K 4096 21.1 us against 10.1), and it is then

@@ -244,8 +244,6 @@ stark_qmm_status launch_moe_adjust(uint32_t* ids, float* weights, const float* s
                                    uint32_t experts, uint32_t active, uint32_t sort_ids, hipStream_t stream);
 // Dense small-M kernel: 4-bit, group 64, M = 9 .. 16, K % 1024 == 0 (qmv_small_m.hip).
 bool small_m_eligible(const AffineOp* ops, uint32_t count);
-// Whether a launch of these products gives every resident workgroup long runs.
-bool small_m_long(const AffineOp* ops, uint32_t count);
 stark_qmm_status launch_small_m(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream);
 // Products of 1 to 16 rows, group 64, any K % 64 == 0, N and plane layout (qmv_dense.hip).
 bool dense_eligible(const AffineOp& op, int bits);

@@ -361,7 +361,7 @@ DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
     }
     if (!few.empty()) few_rows = few_rows_rule(few.data(), (uint32_t)few.size(), bits, cus(), readable);
     if (!many.empty() && small_m_eligible(many.data(), (uint32_t)many.size()))
-        many_rows = !small_m_long(many.data(), (uint32_t)many.size());
+        many_rows = !small_m_long(many.data(), (uint32_t)many.size(), cus());
     if (!mid.empty() && mid_readable) mid_rows = !w8_rows5_mfma(mid.data(), (uint32_t)mid.size(), cus());
 }
 

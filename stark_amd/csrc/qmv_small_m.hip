@@ -331,22 +331,6 @@ bool small_m_eligible(const AffineOp* ops, uint32_t count) {
     return count > 0;
 }
 
-// The dense products' cost that this kernel saves is the activation stage of
-// each 32 rows, through its runs; those need work for many passes per
-// workgroup (16 rows: 11.5 passes per resident workgroup on the Qwen3-8B layer
-// set, 154 us for four layers against 169; 5.9 at hidden 3072 / 8192, 109
-// against 106; 2.2 at hidden 2048 / 6144, 87 against 62).
-bool small_m_long(const AffineOp* ops, uint32_t count) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return false;
-    uint64_t units = 0;
-    for (uint32_t i = 0; i < count; ++i)
-        units += (uint64_t)((ops[i].n + kRows * kSmTiles - 1) / (kRows * kSmTiles)) * (ops[i].k / kSmPass);
-    return units >= 8 * 2 * (uint64_t)cus;
-}
-
 stark_qmm_status launch_small_m(const AffineOp* ops, uint32_t count, bool signed_codes, hipStream_t stream) {
     if (count > (uint32_t)kMaxBatchOps) return STARK_QMM_INVALID_ARGUMENT;  // the batch holds kMaxBatchOps
     int dev = 0, cus = 0;

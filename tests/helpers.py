@@ -95,3 +95,17 @@ def dequant_magnitude(O, codes, scales, corr, n, k, bits, gs, layout, correction
         return mag[:, :n]
     gi = np.asarray(gather).reshape(m, out_n if out_n is not None else n)
     return np.take_along_axis(mag, np.minimum(gi, rows - 1), axis=1)
+
+
+LONG_LAUNCH = (32768, 4096)  # n, k: with such a product beside it, a launch of 9 to 16 rows is long enough for qmv_small_m
+
+
+def long_launch(Q, m, w_dt=BF16, d_dt=BF16):
+    """A 4-bit product of m rows (of zeros) that makes the launch it is in a long one."""
+    import torch
+    n, k = LONG_LAUNCH
+    planes = torch.zeros(n * (k // 64), dtype=torch.int16, device="cuda")
+    return Q.MatmulArguments(a=torch.zeros(m * k, dtype=torch.int16, device="cuda"), m=m, n=n, k=k,
+                             d=torch.zeros(m * n, dtype=torch.float32 if d_dt == F32 else torch.int16, device="cuda"),
+                             b=Q.QuantizedB(codes=torch.zeros(n * k // 2, dtype=torch.uint8, device="cuda"), scales=planes,
+                                            correction_data=planes, params=Q.QuantParams(1, n, k // 64)))

@@ -4,8 +4,10 @@ for, and at the measured sizes the rule takes the faster side."""
 import pytest
 
 from tests import dispatch as D
+from tests import helpers as H
 from tests import test_gpu_a8_dense as A8
 from tests import test_gpu_affine_dense as AD
+from tests import test_gpu_small_m as SM
 
 
 def test_a8_shape_cases_reach_every_shape():
@@ -98,3 +100,13 @@ def test_w8_cases_reach_both_kernels():
     for m, n, k, mfma in AD.W8_ROWS:
         assert 5 <= m <= 8 and D.w8_rows5_mfma([(m, n, k)]) == mfma, (m, n, k)
     assert {c[-1] for c in AD.W8_ROWS} == {True, False}
+
+
+def test_small_m_cases_run_in_long_launches():
+    """And only there: the same sizes alone are the dense kernel's."""
+    for m in SM.ROWS:
+        for n, k in SM.SHAPES:
+            assert 9 <= m <= 16 and n >= 16 and k % 1024 == 0
+            assert D.small_m_long([(m, n, k), (m,) + H.LONG_LAUNCH]) and not D.small_m_long([(m, n, k)])
+    layer = _layer(16, 4096, 12288)
+    assert D.small_m_long(layer) and not D.small_m_long(_layer(16, 3072, 8192)) and not D.small_m_long(_layer(16, 2048, 6144))

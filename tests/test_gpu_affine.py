@@ -28,7 +28,7 @@ def torch_empty(n, dt):
 
 def run_case(Q, O, *, m, n, k, bits=4, gs=64, layout=0, correction=1, w_dt=H.BF16, x_dt=H.BF16, d_dt=H.BF16,
              signed=False, gather=None, bank_rows=None, ab_scale=1.0, accumulate=False, with_bias=False,
-             soft_cap=None, seed=0, quantizer=True, label=""):
+             soft_cap=None, seed=0, quantizer=True, label="", long_launch=False):
     rng = np.random.default_rng(seed)
     rows = n if bank_rows is None else bank_rows
     W = H.affine_weights(O, rng, rows, k, bits, gs, layout, correction, w_dt, quantizer=quantizer)
@@ -53,7 +53,10 @@ def run_case(Q, O, *, m, n, k, bits=4, gs=64, layout=0, correction=1, w_dt=H.BF1
                                  bias=None if bias is None else H.to_dev(bias), soft_cap=soft_cap),
         gather_indices=None if gather is None else H.to_dev(np.asarray(gather, np.uint32)))
     kern = Q.MatmulKernel(w_dt, x_dt, d_dt)
-    kern.encode(args)
+    if long_launch:
+        kern.encode_many([args, H.long_launch(Q, m, w_dt, d_dt)])
+    else:
+        kern.encode(args)
     torch.cuda.synchronize()
     got = H.load(O, H.from_dev(d, np_dtype(d_dt)), d_dt)
     mag = H.dequant_magnitude(O, W["codes"], W["scales"], W["corr"], rows, k, bits, gs, layout, correction, w_dt, x,
@@ -412,26 +415,26 @@ def test_matrix_core_kernel_shapes(qmm, oracle, n, k, gs, m, layout):
 @pytest.mark.parametrize("n,k", [(16, 1024), (40, 4096), (1000, 2048), (96, 12288)])
 @pytest.mark.parametrize("m", [3, 4, 5, 8, 9, 12, 16])
 @pytest.mark.parametrize("layout", [0, 1])
-def test_small_m_dense_kernel_shapes(qmm, oracle, n, k, m, layout):
-    """M = 3 .. 16, 4-bit, group 64, K % 1024 == 0 takes the dense small-M
-    kernel (all 16 activation rows per MFMA, two 16-row tiles per step): one
-    tile, a pair with a shifted second tile, ragged N, long K."""
+def test_dense_kernel_shapes(qmm, oracle, n, k, m, layout):
+    """M = 3 .. 16, 4-bit, group 64 on qmv_dense: whole passes of 1024 values,
+    half a tile of 32 columns, ragged N, long K (launches long enough for
+    qmv_small_m: test_gpu_small_m.py)."""
     run_case(qmm, oracle, m=m, n=n, k=k, gs=64, layout=layout, seed=n + k + 3 * m + layout)
 
 
 @pytest.mark.parametrize("correction,signed,w_dt", [(0, False, H.BF16), (1, True, H.F16), (0, True, H.F16)])
-def test_small_m_dense_kernel_corrections(qmm, oracle, correction, signed, w_dt):
+def test_dense_kernel_corrections(qmm, oracle, correction, signed, w_dt):
     run_case(qmm, oracle, m=11, n=72, k=2048, gs=64, correction=correction, signed=signed, w_dt=w_dt,
              seed=17 + correction + 2 * signed)
 
 
-def test_small_m_dense_kernel_d_ops(qmm, oracle):
+def test_dense_kernel_d_ops(qmm, oracle):
     run_case(qmm, oracle, m=16, n=40, k=1024, gs=64, ab_scale=0.75, accumulate=True, with_bias=True,
              soft_cap=30.0, seed=5)
 
 
-def test_small_m_dense_kernel_batch_matches_single(qmm, oracle):
-    """Three dense-eligible ops (N = 48, 17, 64) in one launch give the bits
+def test_dense_kernel_batch_matches_single(qmm, oracle):
+    """Three products (N = 48, 17, 64) in one launch of qmv_dense give the bits
     of three single launches (the op search by first block)."""
     rng = np.random.default_rng(31)
     k = qmm.MatmulKernel(H.BF16, H.BF16, H.BF16)
@@ -459,19 +462,16 @@ def test_small_m_dense_kernel_batch_matches_single(qmm, oracle):
 
 @pytest.mark.parametrize("n,k", [(9000, 4096), (32010, 1024)])
 @pytest.mark.parametrize("m", [8, 16])
-def test_small_m_dense_kernel_runs(qmm, oracle, n, k, m):
-    """Launches with more tile pairs than resident workgroups: a workgroup
-    runs several pairs pass by pass (three at N = 9000, K = 4096; two at
-    N = 32010, K = 1024, whose last run holds one pair with a shifted tile)."""
+def test_dense_kernel_large(qmm, oracle, n, k, m):
+    """Launches with more tiles than CUs (N = 9000) and than resident workgroups (N = 32010), ragged N."""
     run_case(qmm, oracle, m=m, n=n, k=k, gs=64, layout=1, seed=n + k + m)
 
 
 @pytest.mark.parametrize("variant", ["symmetric", "f16_planes", "signed", "output_group", "m3", "d_ops"])
-def test_small_m_dense_kernel_runs_variants(qmm, oracle, variant):
-    """The multi-pair runs (N = 9000, K = 4096: three pairs per workgroup)
-    with each plane, code and output variant: symmetric codes (no bias
-    plane), f16 planes, signed codes, per-row planes, an odd M, and the
-    D-ops on a run's shifted last tile."""
+def test_dense_kernel_large_variants(qmm, oracle, variant):
+    """N = 9000, K = 4096 with each plane, code and output variant: symmetric
+    codes (no bias plane), f16 planes, signed codes, per-row planes, an odd M,
+    and the D-ops on the ragged last tile."""
     kw = dict(m=8, n=9000, k=4096, gs=64, layout=1, seed=300 + len(variant))
     kw.update({"symmetric": dict(correction=0), "f16_planes": dict(w_dt=H.F16), "signed": dict(signed=True),
                "output_group": dict(layout=0), "m3": dict(m=3),
@@ -479,10 +479,8 @@ def test_small_m_dense_kernel_runs_variants(qmm, oracle, variant):
     run_case(qmm, oracle, **kw)
 
 
-def test_small_m_dense_kernel_run_length_keeps_bits(qmm, oracle):
-    """A K = 12288 product and a K = 4096 product in one launch run one pair
-    per workgroup; alone, the K = 4096 product runs three. Every output row
-    keeps its bits."""
+def test_dense_kernel_depths_keep_bits(qmm, oracle):
+    """A K = 12288 product and a K = 4096 product in one launch and alone: every output row keeps its bits."""
     rng = np.random.default_rng(37)
     k = qmm.MatmulKernel(H.BF16, H.BF16, H.BF16)
     made = []

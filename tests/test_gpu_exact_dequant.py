@@ -74,9 +74,10 @@ def _mode(Q, bits):
 
 
 def _affine_exact(Q, O, *, n, k, m, bits=4, gs=64, layout=1, correction=1, signed=False, w_dt=H.BF16, x_dt=H.BF16,
-                  ncols=40, seed=0, label=""):
+                  ncols=40, seed=0, label="", long_launch=False):
     """Columns in chunks of m one-hot rows; M = 1 chunks go through
-    encode_many (eight products per call, shared weights)."""
+    encode_many (eight products per call, shared weights). long_launch: all
+    chunks in one call with a product that makes it long enough for qmv_small_m."""
     rng = np.random.default_rng(seed)
     codes, s, b = _weights(O, rng, n, k, bits, gs, layout, correction, w_dt)
     cols = _columns(rng, k, ncols)
@@ -105,7 +106,9 @@ def _affine_exact(Q, O, *, n, k, m, bits=4, gs=64, layout=1, correction=1, signe
         outs.append(d)
         args.append(a)
     kern = Q.MatmulKernel(w_dt, x_dt, H.F32)
-    if m == 1:
+    if long_launch:
+        kern.encode_many(args + [H.long_launch(Q, m, w_dt, H.F32)])
+    elif m == 1:
         for i in range(0, len(args), 8):
             kern.encode_many(args[i:i + 8])
     else:
@@ -164,18 +167,32 @@ def test_mfma_8bit_signed_symmetric_exact(qmm, oracle, signed, correction):
                   seed=90 + signed, label="qmv_mfma w8 variants")
 
 
-# ------------------------------------------------------------ qmv_small_m (dense form, M = 3..16)
+# ------------------------------------------------------------ qmv_dense, 4-bit (M = 3..16)
 
 @pytest.mark.parametrize("m", [3, 4, 5, 8, 16])
 @pytest.mark.parametrize("layout", [0, 1])
+def test_dense_exact(qmm, oracle, m, layout):
+    _affine_exact(qmm, oracle, n=96, k=4096, m=m, layout=layout, ncols=32, seed=100 + m + layout,
+                  label=f"qmv_dense m{m}")
+
+
+def test_dense_signed_symmetric_exact(qmm, oracle):
+    _affine_exact(qmm, oracle, n=48, k=2048, m=8, correction=0, signed=True, ncols=16, seed=120,
+                  label="qmv_dense signed symmetric")
+
+
+# ------------------------------------------------------------ qmv_small_m (M = 9..16, long launches)
+
+@pytest.mark.parametrize("m", [9, 16])
+@pytest.mark.parametrize("layout", [0, 1])
 def test_small_m_exact(qmm, oracle, m, layout):
     _affine_exact(qmm, oracle, n=96, k=4096, m=m, layout=layout, ncols=32, seed=100 + m + layout,
-                  label=f"qmv_small_m m{m}")
+                  label=f"qmv_small_m m{m}", long_launch=True)
 
 
 def test_small_m_signed_symmetric_exact(qmm, oracle):
-    _affine_exact(qmm, oracle, n=48, k=2048, m=8, correction=0, signed=True, ncols=16, seed=120,
-                  label="qmv_small_m signed symmetric")
+    _affine_exact(qmm, oracle, n=48, k=2048, m=12, correction=0, signed=True, ncols=16, seed=120,
+                  label="qmv_small_m signed symmetric", long_launch=True)
 
 
 # ------------------------------------------------------------ other GEMV kernels
