@@ -79,6 +79,18 @@ inline bool a8_wave_per_row(uint32_t m, uint32_t n, uint32_t k, int bits, uint32
     return weights <= (k <= 1024 ? 14 : 8) * unit;
 }
 
+// ---- Routed experts: whether a call of group-64 banks takes the grouped products
+// of a prompt (moe_group.hip), whose workgroups are 128 up rows by 64 routes of
+// one expert. From 17 tokens on (us against the slot form of fewer tokens, model /
+// hidden / experts / active: 17 tokens, 2048/768/128/8 77 against 156, 1024/512/
+// 128/2 29 and 38, 2048/512/32/2 33 and 48, 512/512/2/2 25 and 31, 256/128/4/1 17
+// and 29), but for one expert of up to 64 tokens, which is one slot on a few
+// workgroups (2048/1024: 24 tokens 42.8 against 32.5, 64 64.3 and 57.6; 128 65.8 and
+// 100.8), unless it is small (512/256: 21 to 32 against 29 to 36).
+inline bool moe_grouped(uint32_t tokens, uint32_t experts, uint32_t model, uint32_t hidden) {
+    return tokens > 16 && (experts > 1 || tokens > 64 || (uint64_t)model * hidden <= 384 * 1024);
+}
+
 // ---- Products of up to 16 rows, group 64: qmv_dense (32-column tiles, two
 // workgroups per CU, 1024 values a pass) or qmv_mfma (16-column tiles, three per
 // CU, in 64-column groups dealt to the XCDs). Over the products of one launch.

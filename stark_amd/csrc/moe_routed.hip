@@ -824,7 +824,7 @@ stark_qmm_status routed_run(const stark_qmm_routed_args* a, uint8_t* ws, uint64_
     // 38.3; 256 experts 39.3 vs 49.1)
     const bool one = R == 1 && E <= kOneTokenExperts && (uint64_t)A * H * E <= kOneTokenWork;
     // prompts on group-64 banks: slots of up to 64 routes (moe_group.hip)
-    const bool wide = R > 16 && a->up.group_size == 64 && a->down.group_size == 64;
+    const bool wide = a->up.group_size == 64 && a->down.group_size == 64 && moe_grouped(R, E, model, H);
     if (one) {
         RouteOneArgs ra{a->router_logits, a->expert_scales, E, A, a->round_weights_bf16, a->round_logits_bf16,
                         (uint32_t)adjust, sort, ids, weights, table, header};

@@ -7,6 +7,7 @@ from tests import dispatch as D
 from tests import helpers as H
 from tests import test_gpu_a8_dense as A8
 from tests import test_gpu_affine_dense as AD
+from tests import test_gpu_moe_group as MG
 from tests import test_gpu_small_m as SM
 
 
@@ -110,3 +111,10 @@ def test_small_m_cases_run_in_long_launches():
             assert D.small_m_long([(m, n, k), (m,) + H.LONG_LAUNCH]) and not D.small_m_long([(m, n, k)])
     layer = _layer(16, 4096, 12288)
     assert D.small_m_long(layer) and not D.small_m_long(_layer(16, 3072, 8192)) and not D.small_m_long(_layer(16, 2048, 6144))
+
+
+def test_moe_rule():
+    for rows, model, hidden, experts, *_ in MG.SLOTS + MG.EXACT + [(60, 256, 192, 3)]:
+        assert D.moe_grouped(rows, experts, model, hidden)
+    assert not D.moe_grouped(33, 1, 1024, 512) and not D.moe_grouped(64, 1, 1024, 512)
+    assert not D.moe_grouped(16, 128, 2048, 768) and D.moe_grouped(17, 2, 2048, 768) and D.moe_grouped(65, 1, 2048, 1024)

@@ -15,20 +15,29 @@ from tests.moe_cases import case
 pytestmark = pytest.mark.gpu
 
 
+SLOTS = [(17, 256, 192, 8, 2, True), (40, 64, 64, 2, 2, True), (70, 320, 64, 2, 1, False),
+         (150, 192, 320, 3, 2, True), (49, 512, 576, 1, 1, True)]
+EXACT = [(20, 320, 192, 4), (130, 256, 128, 2), (48, 640, 448, 1)]
+
+
 @pytest.mark.parametrize("layout", [0, 1])
-@pytest.mark.parametrize("rows,model,hidden,experts,active,biased",
-                         [(17, 256, 192, 8, 2, True), (40, 64, 64, 2, 2, True), (70, 320, 64, 2, 1, False),
-                          (150, 192, 320, 3, 2, True), (49, 512, 576, 1, 1, True)])
+@pytest.mark.parametrize("rows,model,hidden,experts,active,biased", SLOTS)
 def test_prompt_slots(qmm, oracle, rows, model, hidden, experts, active, biased, layout):
     c = case(oracle, 31 * rows + model + layout, rows, model, hidden, experts, active, layout=layout, biased=biased)
     G.routed_check(qmm, oracle, c)
 
 
 @pytest.mark.parametrize("layout", [0, 1])
-@pytest.mark.parametrize("rows,model,hidden,experts", [(20, 320, 192, 4), (130, 256, 128, 2), (48, 640, 448, 1)])
+@pytest.mark.parametrize("rows,model,hidden,experts", EXACT)
 def test_prompt_products_exact(qmm, oracle, rows, model, hidden, experts, layout):
     X.test_routed_up_product_exact(qmm, oracle, rows, model, hidden, experts, layout)
     X.test_routed_down_product_exact(qmm, oracle, rows, model, hidden, experts, layout)
+
+
+@pytest.mark.parametrize("rows", [33, 64])
+def test_one_expert_of_few_tokens(qmm, oracle, rows):
+    """Left to the slot form by the rule."""
+    G.routed_check(qmm, oracle, case(oracle, rows, rows, 1024, 512, 1, 1, layout=1, biased=True))
 
 
 def test_prompt_signed_codes(qmm, oracle):
