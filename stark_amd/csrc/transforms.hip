@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) void gated_act_mul(GatedArgs a) {
     st8(a.fp_out, a.t_dt, batch * a.gated_dim + k, a.vec_out, v);
 }
 
-// Rows of no whole number of 8 values (no RHT there): thread = one value.
+// Few values, or rows of no whole number of 8 (no RHT): thread = one value.
 __global__ __launch_bounds__(256) void gated_act_mul_one(GatedArgs a) {
     const uint32_t item = blockIdx.x * 256 + threadIdx.x;
     if (item >= a.batch * a.gated_dim) return;
@@ -387,7 +387,15 @@ stark_qmm_status run_transform(TransformArgs a, uint32_t sg, hipStream_t stream)
 
 stark_qmm_status run_gated(GatedArgs a, uint32_t sg, hipStream_t stream) {
     const size_t esz = a.t_dt == STARK_QMM_F32 ? 4 : 2;
-    const bool rows8 = a.gated_dim % kVec == 0;
+    // One value a thread where 8 a thread leave the chip waiting for the divisions
+    // and exponentials of one after the other: no RHT, up to 3072 values a CU (bf16
+    // SiLU of 4096-value rows: 1 row 2.8 against 4.6 us, 128 rows 4.1 and 4.9, 192 rows
+    // 5.0 and 5.1, 256 rows 6.1 and 5.1), and rows of no whole 8 values.
+    int dev = 0, cus = 0;
+    QMM_HIP_CHECK(hipGetDevice(&dev));
+    QMM_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const bool rows8 = a.gated_dim % kVec == 0 &&
+                       (a.factors || (uint64_t)a.batch * a.gated_dim > 3072ull * (uint64_t)cus);
     a.vec_in = aligned(a.act, 16) && aligned(a.factors, 16) &&
                (!a.value || (aligned((const uint8_t*)a.value + (size_t)a.value_offset * esz, 16) &&
                              a.value_row_stride * esz % 16 == 0));

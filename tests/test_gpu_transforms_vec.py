@@ -100,9 +100,21 @@ def test_product_rht_bias_types(qmm, oracle, family, shift, d_dt, w_dt):
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("gated,offset,stride", [(40, 0, 40), (33, 5, 50), (64, 3, 80), (64, 8, 96)])
 def test_gated_rows(qmm, oracle, dt, gated, offset, stride):
-    """Separate operands: value rows at an offset and stride of their own."""
+    """Separate operands: value rows at an offset and stride of their own (few values: one a thread)."""
+    _gated(qmm, oracle, dt, 5, gated, offset, stride)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("offset,stride", [(0, 4104), (8, 4120), (3, 4109)])
+def test_gated_many_values(qmm, oracle, dt, offset, stride):
+    """Past 3072 values a CU eight a thread, aligned and not."""
+    batch, gated = 200, 4104
+    assert batch * gated > 3072 * torch.cuda.get_device_properties(0).multi_processor_count
+    _gated(qmm, oracle, dt, batch, gated, offset, stride)
+
+
+def _gated(qmm, oracle, dt, batch, gated, offset, stride):
     rng = np.random.default_rng(gated + offset)
-    batch = 5
     gate = rng.normal(0, 2, batch * gated).astype(np.float32)
     value = rng.normal(0, 2, offset + batch * stride).astype(np.float32)
     g, v = H.store(oracle, gate, dt), H.store(oracle, value, dt)
