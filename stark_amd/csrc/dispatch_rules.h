@@ -79,6 +79,23 @@ inline bool a8_wave_per_row(uint32_t m, uint32_t n, uint32_t k, int bits, uint32
     return weights <= (k <= 1024 ? 14 : 8) * unit;
 }
 
+// ---- Sampling: whether a call takes the split form (pieces of a row on several
+// workgroups, in three to seven launches) or the row form (one launch, a
+// workgroup a row, two a CU). us, row and split form:
+//   greedy, 1 to 48 rows: 16384 logits 11.2 to 11.9 and 14.0 to 15.2; 16385 more
+//     than in the split form, 151936 nine times (one row)
+//   greedy, 64 rows: 16385 alike; 96: 24000 alike; 128: 20000 1.24 times longer
+//     split, 32000 0.95; 192 and 256: 24000 1.4 and 1.55, 32000 0.77 and 0.96
+//   greedy, 512 rows (two rounds of scratch slots): 32000 1.54, 65536 1.12
+//   sampled, up to 128 rows: shorter split at every size (256 logits, one row:
+//     temperature 38 and 16, top-p 44 and 29; 4096: 49 and 17, 143 and 89)
+//   sampled, 512 rows with filters: 64 logits 1.3 to 1.5 times longer split, 4096
+//     1.0 to 1.1, 16384 0.8 to 1.0; temperature alone 1.0 to 0.6
+inline bool sample_split(uint32_t vocab, uint32_t rows, bool sampled, bool filters) {
+    if (!sampled) return vocab > (rows <= 64 ? 16384u : rows <= 256 ? 28000u : 80000u);
+    return vocab > 1 && !(filters && rows > 256 && vocab <= 16384);
+}
+
 // ---- Routed experts: whether a call of group-64 banks takes the grouped products
 // of a prompt (moe_group.hip), whose workgroups are 128 up rows by 64 routes of
 // one expert. From 17 tokens on (us against the slot form of fewer tokens, model /

@@ -8,11 +8,11 @@
 // Gumbel noise -ln(-ln u), u from Philox4x32-10; the result is the argmax
 // (ties: lower index), or u32::MAX when no finite logit is left.
 //
-// Two forms. Sampled rows, and greedy rows of more than kSplitGreedy logits, are
-// cut into 4096-logit pieces, one workgroup each, in three to seven short
-// launches (see "Split form" below); shorter greedy rows, and the rare rows
-// the split form hands back, take the row form: one workgroup of 1024 threads
-// per row, in passes over the row:
+// Two forms. Sampled rows, and greedy rows of many logits, are cut into
+// 4096-logit pieces, one workgroup each, in three to seven short launches (see
+// "Split form" below); the other rows (sample_split, dispatch_rules.h), and the
+// rare ones the split form hands back, take the row form: one workgroup of 1024
+// threads per row, in passes over the row:
 //  - the prefix kept by the filters has length L, the minimum of top_k, the
 //    count of logits at or above max + ln(min_p), and for top-p the first
 //    prefix whose mass reaches p. Top-p follows the reference's f32 sums in
@@ -41,6 +41,10 @@ namespace qmm {
 namespace {
 
 constexpr int kST = 1024;  // threads per row
+
+// A second 1024-thread workgroup fits a CU up to 80 scalar registers: at 82, 512
+// greedy rows of 16384 logits took 25.0 us in place of 17.5.
+#define QMM_TWO_PER_CU __attribute__((amdgpu_num_sgpr(80)))
 
 struct SampleArgs {
     const void* logits;
@@ -512,7 +516,7 @@ __device__ void sample_row(const SampleArgs& a, size_t row, SampleLds& s, ExactL
     if (tid == 0) a.out[row] = __builtin_isfinite(gb) ? cand : 0xffffffffu;
 }
 
-__global__ __launch_bounds__(kST) void unified_sampling(SampleArgs a) {
+__global__ __launch_bounds__(kST) QMM_TWO_PER_CU void unified_sampling(SampleArgs a) {
     __shared__ SampleLds s;
     __shared__ ExactLds ex;
     sample_row(a, blockIdx.x, s, ex);
@@ -544,12 +548,7 @@ __global__ __launch_bounds__(kST) void unified_sampling(SampleArgs a) {
 // temperature, no finite logit, a bin of more than kExactCap logits) run the
 // row form in 5 or 7. A slot belongs to its row from the claim to the stage
 // that ends the row, whatever streams, threads or graph replays are in flight.
-// The row form's one launch is the shorter for greedy rows of up to 16384
-// logits (11.2-11.9 us against 14.0-15.2 for the three launches, 1 to 32 rows).
-// Sampled rows took longer in it at every size measured (256 logits, one row:
-// temperature 38 against 16 us, top-p 44 against 29; 4096 logits: 49 against
-// 17, 143 against 89), so only rows of one logit keep it.
-constexpr uint32_t kSplitGreedy = 16384, kSplitSampled = 1;
+// Which calls take it: sample_split (dispatch_rules.h).
 constexpr uint32_t kPiece = 4096;
 constexpr int kPer = kPiece / kST;       // logits per thread
 constexpr uint32_t kBins = 256;
@@ -994,7 +993,9 @@ __global__ __launch_bounds__(kST) void split_end(SampleArgs a) {
 stark_qmm_status launch_split(SampleArgs a, uint32_t batch, hipStream_t stream) {
     const uint32_t words = (a.vocab + 31u) / 32u;
     const bool filters = a.has_top_k || a.has_top_p || a.has_min_p;
-    const bool few = a.has_top_k && a.top_k <= (uint32_t)kExactCap;  // split_select ends every row
+    // split_select ends every row of at most as many kept logits as it has threads (with more, a row whose
+    // bins hold over kExactCap would fall to the row form: top-k 4096 of 8192, 1.4 times its time)
+    const bool few = a.has_top_k && a.top_k <= (uint32_t)kST;
     for (uint32_t r0 = 0; r0 < batch; r0 += kSlots) {
         const uint32_t rows = std::min(kSlots, batch - r0);
         SampleArgs b = a;
@@ -1047,13 +1048,14 @@ stark_qmm_status stark_qmm_unified_sampling(const stark_qmm_sampling_args* args,
     a.dt = x.data_type;
     a.has_temperature = x.has_temperature;
     a.temperature = x.temperature;
-    a.has_top_k = x.has_top_k;
+    a.has_top_k = x.has_top_k && x.top_k < x.vocab_size;  // as many as there are: nothing is filtered
     a.top_k = x.top_k;
     a.has_top_p = x.has_top_p;
     a.top_p = x.top_p;
     a.has_min_p = x.has_min_p;
     a.min_p = x.min_p;
-    if (x.vocab_size > (x.seeds ? kSplitSampled : kSplitGreedy) && x.vocab_size < kNoSlot)
+    const bool filters = a.has_top_k || a.has_top_p || a.has_min_p;
+    if (sample_split(x.vocab_size, x.batch_size, x.seeds != nullptr, filters) && x.vocab_size < kNoSlot)
         return launch_split(a, x.batch_size, (hipStream_t)stream);
     hipLaunchKernelGGL(unified_sampling, dim3(x.batch_size), dim3(kST), 0, (hipStream_t)stream, a);
     QMM_HIP_CHECK(hipGetLastError());

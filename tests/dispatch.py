@@ -27,6 +27,7 @@ int few_rows(const Op* ops, const int* readable, uint32_t count, int bits, uint3
     const qmm::FewRowsRule r = qmm::few_rows_rule(ops, count, bits, cus, read);
     return (r.idle ? 1 : 0) | (r.drag ? 2 : 0);
 }
+int sample_split(uint32_t v, uint32_t rows, int sampled, int filters) { return qmm::sample_split(v, rows, sampled != 0, filters != 0); }
 int moe_grouped(uint32_t t, uint32_t e, uint32_t model, uint32_t hidden) { return qmm::moe_grouped(t, e, model, hidden); }
 int small_m_long(const Op* ops, uint32_t count, uint32_t cus) { return qmm::small_m_long(ops, count, cus); }
 int w8_rows5_mfma(const Op* ops, uint32_t count, uint32_t cus) { return qmm::w8_rows5_mfma(ops, count, cus); }
@@ -80,3 +81,7 @@ def small_m_long(sizes, cus=CUS):
 
 def moe_grouped(tokens, experts, model, hidden):
     return bool(rules().moe_grouped(tokens, experts, model, hidden))
+
+
+def sample_split(vocab, rows, sampled, filters):
+    return bool(rules().sample_split(vocab, rows, int(sampled), int(filters)))

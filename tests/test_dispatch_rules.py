@@ -118,3 +118,22 @@ def test_moe_rule():
         assert D.moe_grouped(rows, experts, model, hidden)
     assert not D.moe_grouped(33, 1, 1024, 512) and not D.moe_grouped(64, 1, 1024, 512)
     assert not D.moe_grouped(16, 128, 2048, 768) and D.moe_grouped(17, 2, 2048, 768) and D.moe_grouped(65, 1, 2048, 1024)
+
+
+# logits, rows, sampled, filters, time in the split form over that in the row form
+MEASURED_SAMPLE = [(16385, 32, False, False, 0.82), (20000, 48, False, False, 0.79), (151936, 1, False, False, 0.11),
+                   (16385, 128, False, False, 1.38), (24000, 256, False, False, 1.55), (32000, 192, False, False, 0.80),
+                   (32000, 512, False, False, 1.54), (65536, 512, False, False, 1.12), (2, 1, True, False, 0.60),
+                   (64, 512, True, True, 1.43), (4096, 512, True, True, 1.05), (256, 128, True, True, 0.62),
+                   (16384, 512, True, False, 0.60), (4096, 32, True, True, 0.61)]
+
+
+@pytest.mark.parametrize("vocab,rows,sampled,filters,ratio", MEASURED_SAMPLE)
+def test_sampling_rule_takes_the_faster_side(vocab, rows, sampled, filters, ratio):
+    assert D.sample_split(vocab, rows, sampled, filters) == (ratio < 1)
+
+
+def test_sampling_cases_reach_the_split_form():
+    for vocab, batch in [(16385, 3), (20480, 2), (32769, 2), (17000, 4), (81000, 300)]:
+        assert D.sample_split(vocab, batch, False, False) and D.sample_split(vocab, batch, True, True)
+    assert D.sample_split(16400, 300, True, True) and not D.sample_split(600, 300, True, True)

@@ -63,6 +63,28 @@ def test_more_rows_than_slots(qmm, oracle):
         _check(qmm, oracle, x, F32, vocab, batch, opts)
 
 
+def test_more_greedy_rows_than_slots(qmm, oracle):
+    x = np.random.default_rng(18).normal(0, 2, 300 * 81000).astype(np.float32)
+    _check(qmm, oracle, x, F32, 81000, 300, None)
+
+
+@pytest.mark.parametrize("vocab", [2, 33, 600])
+def test_many_short_rows(qmm, oracle, vocab):
+    """Past 256 rows, short filtered rows take the row form; top-k of all logits filters nothing."""
+    x = np.random.default_rng(vocab).normal(0, 2, 300 * vocab).astype(np.float32)
+    for opts in (None, dict(temperature=0.8), dict(temperature=0.8, top_k=vocab), dict(top_k=vocab, top_p=0.9),
+                 dict(top_k=max(1, vocab // 2)), dict(temperature=2.0, top_p=0.7, min_p=0.1)):
+        _check(qmm, oracle, x, F32, vocab, 300, opts)
+
+
+@pytest.mark.parametrize("vocab,top_k", [(4096, 1024), (4096, 1025), (8192, 4096), (20000, 3000)])
+def test_large_top_k(qmm, oracle, vocab, top_k):
+    """Both sides of the size up to which the sorting stage ends every row."""
+    x = np.random.default_rng(top_k).normal(0, 2, 3 * vocab).astype(np.float32)
+    for opts in (dict(top_k=top_k), dict(top_k=top_k, top_p=0.999, temperature=3.0), dict(top_k=top_k, min_p=1e-4)):
+        _check(qmm, oracle, x, F32, vocab, 3, opts)
+
+
 def test_streams_and_replays(qmm, oracle):
     """Calls on two streams and replays of a captured call in flight together give the tokens of single calls."""
     vocab, batch = 40000, 5
