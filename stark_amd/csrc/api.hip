@@ -212,7 +212,7 @@ stark_qmm_status encode_product(stark_qmm_kernel* kr, const stark_qmm_args* args
     // the reference's Metal GEMM); the reference-accumulation mode keeps the
     // f32-dequant GEMV kernels for every M (kernel.rs:34-37, metal mod.rs:341-357).
     if (!kr->reference_accumulation && !materialize && gemm_stream_eligible(op, bits) &&
-        (op.m <= 64 || gemm_stream_pays(&op, 1)))
+        (op.m <= 64 || gemm_stream_pays(&op, 1, bits)))
         return launch_gemm_stream(&op, 1, bits, stream);
     if (!kr->reference_accumulation && !materialize && gemm_eligible(op, bits))
         return launch_affine_gemm(op, bits, stream);
@@ -325,7 +325,7 @@ stark_qmm_status stark_qmm_encode_many(stark_qmm_kernel* kr, const stark_qmm_arg
     }
     for (int b8 = 0; b8 < 2; ++b8)
         for (auto& v : streamed[b8]) {
-            if (gemm_stream_pays(v.data(), (uint32_t)v.size())) continue;
+            if (gemm_stream_pays(v.data(), (uint32_t)v.size(), b8 ? 8 : 4)) continue;
             std::vector<AffineOp> keep;
             for (const AffineOp& op : v) {
                 if (op.m > 64)

@@ -79,6 +79,81 @@ inline bool a8_wave_per_row(uint32_t m, uint32_t n, uint32_t k, int bits, uint32
     return weights <= (k <= 1024 ? 14 : 8) * unit;
 }
 
+// ---- Prompt products of 17 to 128 rows, group 64: qgemm_stream, whose workgroups
+// take 32 or 64 columns by one of equal row blocks (at most 64 rows), two a CU, or
+// the GEMM (128 rows by 64 columns, one a CU) past 64 rows.
+
+// 16-row blocks of a workgroup.
+template <class Op>
+uint32_t stream_blocks(const Op* ops, uint32_t count) {
+    uint32_t m = 0;
+    for (uint32_t i = 0; i < count; ++i) m = std::max(m, ops[i].m);
+    const uint32_t blocks = (m + 63) / 64;
+    return std::max(2u, (m + 16 * blocks - 1) / (16 * blocks));
+}
+
+// 64-column workgroups of a launch.
+template <class Op>
+uint64_t stream_tiles(const Op* ops, uint32_t count) {
+    const uint32_t rows = 16 * stream_blocks(ops, count);
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < count; ++i) tiles += (uint64_t)((ops[i].n + 63) / 64) * ((ops[i].m + rows - 1) / rows);
+    return tiles;
+}
+
+// 64 columns a workgroup (each LDS read feeds two matrix products) instead of
+// 32: from 1.5 workgroups a CU on (64 rows of the seven products of 4096 / 12288,
+// 608: 71.9 against 77.9 us; of 2560 / 6912, 356: 37.7 against 32.2; 32 rows, N
+// 20480, K 4096, 320: 29.4 and 29.2, N 28672, 448: 29.9 against 35.6), and with 33
+// rows and more of one depth already where 32 columns make between one and three
+// a CU (64 rows, K 4096: N 8192, 128 workgroups of 64 columns 22.8 against 16.3; N
+// 10240, 160: 22.9 against 26.6; 96 rows, N 10240, 320: 28.9 against 30.4, K 2048
+// 17.5 against 16.1). With few columns a workgroup the activations come from L2
+// too often for 25 to 32 rows of a deep product (N 12288, K 12288: 17 rows 42.7 us,
+// 32 rows 52.1, 64 columns 49.9).
+template <class Op>
+bool stream_wide(const Op* ops, uint32_t count, uint32_t cus) {
+    const uint64_t tiles = stream_tiles(ops, count);
+    if (2 * tiles > 3 * (uint64_t)cus) return true;
+    uint32_t k = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (ops[i].k != ops[0].k) return false;
+        k = ops[i].k;
+    }
+    return stream_blocks(ops, count) > 2 && 2 * tiles > cus && (tiles <= cus || k > 2048);
+}
+
+// Whether a launch's products of more than 64 rows run on qgemm_stream. One
+// depth: by its 64-column workgroups a CU. The GEMM's tiles are as many as half
+// of them, and full past 112 rows. us, GEMM and here, K 4096, 4-bit: 97 rows, N 8192
+// (1.0) 32.4 22.5, 10240 (1.25) 32.6 30.5, 12288 (1.5) 32.7 34.3, 28672 50.9 64.1; 96
+// rows, 12288 32.7 31.9, 16384 (2.0) 33.5 32.6 (8-bit, K 12288: 100.7 104.8), 20480
+// (2.5) 48.6 46.4 (K 1024: 16.3 16.9), 28672 (3.5) 51.1 58.5; 128 rows, 8192 30.9 22.9, 10240 31.2 31.7
+// (8-bit 35.0 32.6, K 2048 19.6 19.9), 12288 31.4 36.3. Several depths: the GEMM
+// takes what its deepest product's serial K loop takes, about 7.8 ns a value of K,
+// or, with tiles enough, 0.5 us for 2^20 weights, where this kernel takes 0.55:
+// here from 62 values of K for 10^6 weights (97 rows, seven products: 1024 / 1024
+// (176) 13.9 and 10.0, 2560 / 6912 (99) 53 and 44, 4096 / 12288 (64) 103.5 and 100,
+// 4096 / 8192 (57) 73.6 and 81.5), past 112 rows with a deep product only (128 rows
+// of 1536 / 1536 (118) 15.6 and 16.9, 2048 / 2048 (89) 19.3 and 21.2).
+template <class Op>
+bool stream_takes(const Op* ops, uint32_t count, int bits, uint32_t cus) {
+    double weights = 0, k = 0;
+    uint32_t m = 0;
+    bool mixed = false;
+    for (uint32_t i = 0; i < count; ++i) {
+        weights += 1e-6 * ops[i].n * ops[i].k;
+        k = std::max(k, (double)ops[i].k);
+        m = std::max(m, ops[i].m);
+        mixed = mixed || ops[i].k != ops[0].k;
+    }
+    if (mixed) return k >= 62 * weights && (m <= 112 || k >= 2816 || k >= 150 * weights);
+    const double fill = (double)stream_tiles(ops, count) / cus;
+    if (m <= 96) return fill <= 1.5 || (fill > 2.0 && fill <= 2.5 && k > 1024);
+    if (m <= 112) return fill <= (k > 2048 ? 1.25 : 1.0);
+    return fill <= (k > 512 ? 1.0 : 0.75) || (bits == 8 && fill <= 1.25 && k > 2048);
+}
+
 // ---- Sampling: whether a call takes the split form (pieces of a row on several
 // workgroups, in three to seven launches) or the row form (one launch, a
 // workgroup a row, two a CU). us, row and split form:

@@ -306,34 +306,19 @@ bool gemm_stream_eligible(const AffineOp& o, int bits) {
             (uint64_t)64 * o.k * 2 < (1ull << 31));
 }
 
-// Whether a launch's products of more than 64 rows (all of them gemm_eligible)
-// run here; those of up to 64 always do. The GEMM then takes what its deepest
-// product's serial K loop takes, about 7.8 ns a value of K, or, with tiles enough, 0.5 us for 2^20
-// weights, where this kernel takes 0.55: here from 62 values of K for 10^6
-// weights. us of a 4-bit layer at 97 rows (values of K for 10^6 weights), GEMM
-// and here: 1024/1024 (176) 13.9 and 10.0, 2560/6912 (99) 53 and 44, 4096/12288
-// (64) 103.5 and 100, 3072/3072 (59) 38.2 and 38.2, 4096/8192 (57) 73.6 and 81.5,
-// 4096/6144 (49) 61.3 and 71.3. Past 112 rows the GEMM's tiles are full and
-// short launches without a deep product stay with it: 128 rows of 1536/1536 (118)
-// 15.6 and 16.9, 2048/2048 (89) 19.3 and 21.2.
-bool gemm_stream_pays(const AffineOp* ops, uint32_t count) {
-    double weights = 0, k = 0;
-    uint32_t m = 0;
-    for (uint32_t i = 0; i < count; ++i) {
-        if (ops[i].m <= 64) continue;
-        weights += 1e-6 * ops[i].n * ops[i].k;
-        k = std::max(k, (double)ops[i].k);
-        m = std::max(m, ops[i].m);
-    }
-    return k >= 62 * weights && (m <= 112 || k >= 2816 || k >= 150 * weights);
+bool gemm_stream_pays(const AffineOp* ops, uint32_t count, int bits) {
+    std::vector<AffineOp> tall;
+    for (uint32_t i = 0; i < count; ++i)
+        if (ops[i].m > 64) tall.push_back(ops[i]);
+    int dev = 0, cus = 0;
+    if (tall.empty() || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return tall.empty();
+    return stream_takes(tall.data(), (uint32_t)tall.size(), bits, (uint32_t)cus);
 }
 
 // ops: all gemm_stream_eligible for `bits`, of one plane type; longest K first.
-// Row blocks of equal size, at most 64 rows each. 64 columns a workgroup (each
-// LDS read feeds two matrix products) from 1.5 workgroups a CU, else 32: 64 rows
-// of 2560/6912 (356 workgroups of 64 columns) 32.2 us with 32 columns and 37.7
-// with 64, of 4096/12288 (608) 77.9 and 71.9; 128 rows of 1984/2560 (406) 25.3
-// and 21.7.
+// Row blocks of equal size, at most 64 rows each; 32 or 64 columns a workgroup (stream_wide).
 stark_qmm_status launch_gemm_stream(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream) {
     if (count == 0) return STARK_QMM_OK;
     if (count > (uint32_t)kMaxBatchOps) return STARK_QMM_UNSUPPORTED;
@@ -341,16 +326,11 @@ stark_qmm_status launch_gemm_stream(const AffineOp* ops, uint32_t count, int bit
     std::copy(ops, ops + count, b.op);
     std::stable_sort(b.op, b.op + count, [](const AffineOp& x, const AffineOp& y) { return x.k > y.k; });
     b.count = count;
-    uint32_t mmax = 0;
-    for (uint32_t i = 0; i < count; ++i) mmax = std::max(mmax, ops[i].m);
-    const uint32_t blocks = (mmax + 63) / 64, mt = std::max(2u, (mmax + 16 * blocks - 1) / (16 * blocks));
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < count; ++i)
-        tiles += (uint64_t)((ops[i].n + 63) / 64) * ((ops[i].m + 16 * mt - 1) / (16 * mt));
+    const uint32_t mt = stream_blocks(ops, count);
     int dev = 0, cus = 0;
     QMM_HIP_CHECK(hipGetDevice(&dev));
     QMM_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const bool wide = 2 * tiles > 3 * (uint64_t)cus;
+    const bool wide = stream_wide(ops, count, (uint32_t)cus);
     if (mt == 2) return wide ? launch_shape<2, 2>(b, bits, stream) : launch_shape<2, 1>(b, bits, stream);
     if (mt == 3) return wide ? launch_shape<3, 2>(b, bits, stream) : launch_shape<3, 1>(b, bits, stream);
     return wide ? launch_shape<4, 2>(b, bits, stream) : launch_shape<4, 1>(b, bits, stream);

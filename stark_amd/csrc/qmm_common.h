@@ -237,7 +237,8 @@ stark_qmm_status launch_affine_gemm(const AffineOp& op, int bits, hipStream_t st
 stark_qmm_status launch_affine_gemm_group(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);
 // Weight-streaming kernel for prompts of 17 to 128 rows, group 64 (qgemm_stream.hip).
 bool gemm_stream_eligible(const AffineOp& op, int bits);
-bool gemm_stream_pays(const AffineOp* ops, uint32_t count);  // for its products of more than 64 rows
+// Whether it takes a call's products of more than 64 rows (all of them gemm_eligible; true when there are none).
+bool gemm_stream_pays(const AffineOp* ops, uint32_t count, int bits);
 stark_qmm_status launch_gemm_stream(const AffineOp* ops, uint32_t count, int bits, hipStream_t stream);
 // Route adjustment with optional gains (moe.hip).
 stark_qmm_status launch_moe_adjust(uint32_t* ids, float* weights, const float* scales, uint32_t rows,

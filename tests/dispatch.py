@@ -27,6 +27,9 @@ int few_rows(const Op* ops, const int* readable, uint32_t count, int bits, uint3
     const qmm::FewRowsRule r = qmm::few_rows_rule(ops, count, bits, cus, read);
     return (r.idle ? 1 : 0) | (r.drag ? 2 : 0);
 }
+int stream_wide(const Op* ops, uint32_t count, uint32_t cus) { return qmm::stream_wide(ops, count, cus); }
+int stream_takes(const Op* ops, uint32_t count, int bits, uint32_t cus) { return qmm::stream_takes(ops, count, bits, cus); }
+int stream_blocks(const Op* ops, uint32_t count) { return (int)qmm::stream_blocks(ops, count); }
 int sample_split(uint32_t v, uint32_t rows, int sampled, int filters) { return qmm::sample_split(v, rows, sampled != 0, filters != 0); }
 int moe_grouped(uint32_t t, uint32_t e, uint32_t model, uint32_t hidden) { return qmm::moe_grouped(t, e, model, hidden); }
 int small_m_long(const Op* ops, uint32_t count, uint32_t cus) { return qmm::small_m_long(ops, count, cus); }
@@ -85,3 +88,15 @@ def moe_grouped(tokens, experts, model, hidden):
 
 def sample_split(vocab, rows, sampled, filters):
     return bool(rules().sample_split(vocab, rows, int(sampled), int(filters)))
+
+
+def stream_wide(sizes, cus=CUS):
+    return bool(rules().stream_wide(ops(*sizes), len(sizes), cus))
+
+
+def stream_takes(sizes, bits, cus=CUS):
+    return bool(rules().stream_takes(ops(*sizes), len(sizes), bits, cus))
+
+
+def stream_blocks(sizes):
+    return rules().stream_blocks(ops(*sizes), len(sizes))

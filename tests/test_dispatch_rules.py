@@ -7,6 +7,7 @@ from tests import dispatch as D
 from tests import helpers as H
 from tests import test_gpu_a8_dense as A8
 from tests import test_gpu_affine_dense as AD
+from tests import test_gpu_gemm_stream as GS
 from tests import test_gpu_moe_group as MG
 from tests import test_gpu_small_m as SM
 
@@ -137,3 +138,40 @@ def test_sampling_cases_reach_the_split_form():
     for vocab, batch in [(16385, 3), (20480, 2), (32769, 2), (17000, 4), (81000, 300)]:
         assert D.sample_split(vocab, batch, False, False) and D.sample_split(vocab, batch, True, True)
     assert D.sample_split(16400, 300, True, True) and not D.sample_split(600, 300, True, True)
+
+
+# products of a launch, bits, us on the GEMM and streaming
+MEASURED_STREAM = [([(97, 8192, 4096)], 4, 32.4, 22.5), ([(97, 10240, 4096)], 4, 32.6, 30.5), ([(97, 12288, 4096)], 4, 32.7, 34.3),
+                   ([(97, 28672, 4096)], 4, 50.9, 64.1), ([(96, 12288, 8192)], 4, 59.2, 58.1), ([(96, 20480, 4096)], 4, 48.6, 46.4),
+                   ([(96, 28672, 2048)], 8, 32.0, 36.1), ([(128, 8192, 4096)], 4, 30.9, 22.9), ([(128, 10240, 2048)], 4, 16.1, 19.0),
+                   ([(128, 12288, 8192)], 4, 58.0, 65.6), ([(128, 10240, 8192)], 8, 66.0, 58.3), ([(128, 12288, 4096)], 8, 35.5, 38.0),
+                   (_pair(100, 2048, 6144), 4, 18.6, 19.1), (_pair(128, 2048, 6144), 8, 17.4, 19.2), (_pair(100, 2560, 6912), 4, 21.8, 23.7),
+                   (_layer(100, 4096, 12288), 4, 104.0, 100.0), (_layer(97, 2560, 6912), 4, 53.0, 44.0),
+                   (_layer(97, 4096, 8192), 4, 73.6, 81.5), (_layer(128, 2048, 2048), 4, 19.3, 21.2)]
+
+
+@pytest.mark.parametrize("sizes,bits,gemm,stream", MEASURED_STREAM)
+def test_stream_rule_takes_the_faster_side(sizes, bits, gemm, stream):
+    assert D.stream_takes(sizes, bits) == (stream < gemm)
+
+
+# products of a launch, us with 32 and with 64 columns a workgroup
+MEASURED_WIDE = [([(64, 8192, 4096)], 16.3, 22.8), ([(64, 10240, 4096)], 26.6, 22.9), ([(64, 16384, 4096)], 27.3, 23.5),
+                 ([(64, 28672, 4096)], 49.9, 38.9), ([(96, 10240, 2048)], 16.1, 17.5), ([(96, 10240, 4096)], 30.4, 28.9),
+                 ([(48, 12288, 8192)], 43.6, 37.0), ([(17, 10240, 8192)], 28.8, 33.4), ([(32, 28672, 4096)], 35.6, 29.9),
+                 ([(128, 4096, 4096)], 13.9, 20.3), ([(128, 8192, 4096)], 25.4, 22.9), (_layer(64, 2560, 6912), 32.2, 37.7),
+                 (_layer(64, 4096, 12288), 77.9, 71.9)]
+
+
+@pytest.mark.parametrize("sizes,narrow,wide", MEASURED_WIDE)
+def test_stream_width_takes_the_faster_side(sizes, narrow, wide):
+    assert D.stream_wide(sizes) == (wide < narrow)
+
+
+def test_stream_cases_reach_both_widths_and_the_kernel():
+    for m, n, k, f16, wide in GS.SUMS:
+        assert D.stream_wide([(m, n, k)]) == wide, (m, n, k)
+        assert m <= 64 or D.stream_takes([(m, n, k)], 4)
+    for m, n, k in GS.EXACT:
+        assert m <= 64 or (D.stream_takes([(m, n, k)], 4) and D.stream_takes([(m, n, k)], 8)), (m, n, k)
+    assert {D.stream_blocks([(m, n, k)]) for m, n, k in GS.EXACT} == {2, 3, 4}

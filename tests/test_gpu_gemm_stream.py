@@ -15,9 +15,16 @@ from tests import test_gpu_exact_dequant as E
 pytestmark = pytest.mark.gpu
 
 
+EXACT = [(17, 1, 64), (32, 33, 192), (33, 40, 320), (48, 97, 576), (49, 31, 1088), (64, 65, 2112), (65, 100, 832), (96, 17, 256),
+         (97, 70, 1216), (128, 33, 512)]
+# m, n, k, f16 planes and results; 64 columns a workgroup (else 32)
+SUMS = [(20, 3000, 448, False, False), (40, 25000, 320, True, True), (64, 25000, 192, False, True), (100, 600, 3520, True, False),
+        (128, 600, 4416, False, False), (24, 25000, 320, False, True), (60, 10000, 1088, True, True), (80, 5000, 832, False, True),
+        (128, 8100, 576, False, True)]
+
+
 @pytest.mark.parametrize("bits,layout", [(4, 0), (4, 1), (8, 0), (8, 1)])
-@pytest.mark.parametrize("m,n,k", [(17, 1, 64), (32, 33, 192), (33, 40, 320), (48, 97, 576), (49, 31, 1088), (64, 65, 2112),
-                                   (65, 100, 832), (96, 17, 256), (97, 70, 1216), (128, 33, 512)])
+@pytest.mark.parametrize("m,n,k", EXACT)
 def test_stream_weights_exact(qmm, oracle, bits, layout, m, n, k):
     E._gemm_exact(qmm, oracle, n=n, k=k, bits=bits, layout=layout, seed=m + n + k, m=m, label="qgemm_stream")
 
@@ -28,9 +35,8 @@ def test_stream_corrections_exact(qmm, oracle, correction, signed, bits, m):
     E._gemm_exact(qmm, oracle, n=72, k=1216, bits=bits, correction=correction, signed=signed, seed=m, m=m, label="qgemm_stream")
 
 
-@pytest.mark.parametrize("m,n,k,f16", [(20, 3000, 448, False), (40, 25000, 320, True), (64, 25000, 192, False),
-                                       (100, 600, 3520, True), (128, 600, 4416, False)])
-def test_stream_sums(qmm, oracle, m, n, k, f16):
+@pytest.mark.parametrize("m,n,k,f16,wide", SUMS)
+def test_stream_sums(qmm, oracle, m, n, k, f16, wide):
     """Both column widths against the f64 product of the bf16-effective weights, with the D-ops; f16 planes and results at two sizes."""
     A._skinny_case(qmm, oracle, m, n, k, seed=m + n, ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=30.0,
                    w_dt=H.F16 if f16 else H.BF16, d_dt=H.BF16 if f16 else H.F32)
