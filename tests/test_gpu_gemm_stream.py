@@ -11,6 +11,8 @@ import torch
 from tests import helpers as H
 from tests import test_gpu_affine as A
 from tests import test_gpu_exact_dequant as E
+from tests import test_gpu_range as R
+from tests.tolerances import check
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +91,47 @@ def test_products_past_the_gemm_keep_f32_weights(qmm, n, k, m):
             w = codes[rows].double().view(-1, k // 64, 64) * s[rows].double().unsqueeze(2) + b[rows].double().unsqueeze(2)
             want = x.double() @ w.view(-1, k).t().contiguous()
             assert ((d[:, rows].double() - want).norm() / want.norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(20, 48, 1088), (100, 96, 832)])
+def test_stream_activation_range(qmm, oracle, bits, m, n, k):
+    """Activations of 2^-100 to 2^70, groups of mixed magnitudes and bf16 subnormals, against the f64 product."""
+    rng = np.random.default_rng(m + bits)
+    w = H.affine_weights(oracle, rng, n, k, bits, 64, 1, 1, H.BF16)
+    x = H.store(oracle, R.wide_x(rng, m, k), H.BF16)
+    got = _product(qmm, w, x, m, n, k, bits)
+    want, mag = A.bf16_effective_reference(oracle, w, x, m, n, k, bits, 64, 1, 1, H.BF16, False)
+    check(got.ravel(), want.ravel(), mag=mag.ravel(), label=f"range m{m} b{bits}")
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m", [20, 100])
+def test_stream_non_finite_activations(qmm, oracle, bits, m):
+    """A row with an infinity or a NaN is not finite where its f64 product with
+    the same bf16 weights is not, with that sign; the others keep their bits."""
+    rng = np.random.default_rng(m + bits)
+    n, k = 80, 832
+    w = H.affine_weights(oracle, rng, n, k, bits, 64, 1, 1, H.BF16)
+    xf = rng.normal(0, 1, (m, k)).astype(np.float32)
+    plain = _product(qmm, w, H.store(oracle, xf.ravel(), H.BF16), m, n, k, bits)
+    xf[2, 5], xf[m - 1, k - 3], xf[7, 100] = np.inf, -np.inf, np.nan
+    x = H.store(oracle, xf.ravel(), H.BF16)
+    got = _product(qmm, w, x, m, n, k, bits)
+    with np.errstate(invalid="ignore"):
+        want, _ = A.bf16_effective_reference(oracle, w, x, m, n, k, bits, 64, 1, 1, H.BF16, False)
+    bad = [2, 7, m - 1]
+    assert np.array_equal(np.isnan(got[bad]), np.isnan(want[bad]))
+    inf = np.isinf(want[bad])
+    assert inf.any() and np.array_equal(np.sign(got[bad][inf]), np.sign(want[bad][inf])) and np.isinf(got[bad][inf]).all()
+    rest = np.setdiff1d(np.arange(m), bad)
+    assert np.array_equal(got[rest].view(np.uint32), plain[rest].view(np.uint32))
+
+
+def _product(qmm, w, x, m, n, k, bits):
+    d = torch.zeros(m * n, dtype=torch.float32, device="cuda")
+    qmm.MatmulKernel(H.BF16, H.BF16, H.F32).encode(qmm.MatmulArguments(a=H.to_dev(x), m=m, n=n, k=k, d=d, b=qmm.QuantizedB(
+        codes=H.to_dev(w["codes"]), scales=H.to_dev(w["scales"]), correction_data=H.to_dev(w["corr"]),
+        params=qmm.QuantParams(1, n, k // 64), mode=qmm.MODE_U4 if bits == 4 else qmm.MODE_U8)))
+    torch.cuda.synchronize()
+    return d.cpu().numpy().reshape(m, n)

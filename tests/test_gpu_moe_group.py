@@ -53,3 +53,45 @@ def test_prompt_signed_codes(qmm, oracle):
     torch.cuda.synchronize()
     got = (H.from_dev(out.view(torch.int16), np.uint16).astype(np.uint32) << 16).view(np.float32)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def _by_slots(qmm, c, step=8):
+    """The same tokens, `step` a call: the slot form of few tokens."""
+    rows = []
+    for r in range(0, c["rows"], step):
+        n = min(step, c["rows"] - r)
+        part = dict(c, rows=n, x=c["x"].reshape(c["rows"], -1)[r:r + n].ravel(),
+                    logits=c["logits"].reshape(c["rows"], -1)[r:r + n].ravel())
+        rows.append(G.routed_run(qmm, part).reshape(n, -1))
+    return np.concatenate(rows)
+
+
+def test_prompt_activation_range(qmm, oracle):
+    """Tokens of 2^-100 to 2^50, of mixed magnitudes and of bf16 subnormals: as
+    in the slot form, whose products are the same up to the order of the f32 sums
+    (a bf16 ulp in each of the three stages, of the row's largest value)."""
+    c = case(oracle, 41, 60, 256, 192, 3, 2)
+    rng = np.random.default_rng(41)
+    x = oracle.bf16_to_f32(c["x"]).reshape(60, 256) * np.exp2(rng.integers(-100, 51, (60, 1))).astype(np.float32)
+    x[1::7, :64] *= np.float32(2.0 ** -60)
+    x[5] = rng.integers(1, 127, 256) * 2.0 ** -133
+    c["x"] = oracle.f32_to_bf16(np.ascontiguousarray(x.astype(np.float32).ravel()))
+    got, want = G.routed_run(qmm, c).reshape(60, -1).astype(np.float64), _by_slots(qmm, c).astype(np.float64)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert np.all(np.abs(got - want) <= 3 * 2.0 ** -8 * np.abs(want).max(axis=1, keepdims=True))
+    assert (np.abs(want).max(axis=1) > 0).sum() > 40
+
+
+def test_prompt_non_finite_activations(qmm, oracle):
+    """Infinities and NaN stay in their token, and there as in the slot form: not finite in the same places."""
+    c = case(oracle, 43, 40, 256, 192, 3, 2)
+    x = oracle.bf16_to_f32(c["x"]).reshape(40, 256).copy()
+    plain = G.routed_run(qmm, c).reshape(40, -1)
+    x[3, 70], x[17, 5], x[30, 255], x[38, 0] = np.inf, -np.inf, np.nan, 3.3e38
+    c["x"] = oracle.f32_to_bf16(np.ascontiguousarray(x.ravel()))
+    got, want = G.routed_run(qmm, c).reshape(40, -1), _by_slots(qmm, c)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    touched = [3, 17, 30, 38]
+    assert not np.isfinite(got[[3, 17, 30]]).all()
+    others = np.setdiff1d(np.arange(40), touched)
+    assert np.array_equal(got[others].view(np.uint32), plain[others].view(np.uint32))
