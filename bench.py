@@ -426,7 +426,7 @@ def verify_lines(args, torch, Q, gen, kern, layers, stream):
                    args.warmup, stream)
         nbytes = algorithmic_bytes(m)
         gbs = nbytes / (ms * 1e-3) / 1e9
-        what = ("speculative verify" if m <= 16 else "short prefill, bf16-effective weights" if m <= 64
+        what = ("speculative verify" if m <= 16 else "short prefill, weight-streaming product" if m <= 128
                 else "short prefill, dequant-GEMM")
         emit({"metric": f"q4 matvec HBM GB/s at M={m} ({what})", "value": round(gbs, 1),
                           "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,

@@ -30,4 +30,14 @@ QMM_HOST_DEVICE uint32_t code_offset(uint32_t k, uint32_t h, uint32_t kq, uint32
 QMM_HOST_DEVICE uint32_t code_lane_offset(uint32_t kq, uint32_t K) { return 32 * kq < K ? 16 * kq : 0; }
 QMM_HOST_DEVICE uint32_t code_chunk_offset(uint32_t k, uint32_t kq, uint32_t K) { return k + 32 * kq < K ? k / 2 : 0; }
 
+// Place of 8-value piece v of a pass in MFMA order (what the loads above make of
+// a row). 4-bit: within a 64-value group, piece 4 (kq & 1) + 2 j + (kq >> 1)
+// belongs to lane quarter kq of the group's j-th MFMA (permlane32_swap of 16-byte
+// loads); 8-bit: piece 2 kq + j.
+template <int BITS>
+QMM_HOST_DEVICE uint32_t piece_pos(uint32_t v) {
+    const uint32_t p = v & 7;
+    return (v & ~7u) + (BITS == 4 ? 4 * ((p >> 1) & 1) + ((p >> 2) | ((p & 1) << 1)) : 4 * (p & 1) + (p >> 1));
+}
+
 }  // namespace qmm

@@ -75,7 +75,9 @@ __device__ __forceinline__ float wave_sums(float (&v)[V], int lane) {
 // each output and wave; wave_sums takes 10 for 8 outputs and 32 for 32, most of
 // them lane swaps. A router of 128 rows, K = 2048, at 1, 8, 64, 512 and 2048
 // rows: 3.8, 4.5, 5.8, 23.1, 79 -> 2.4, 2.7, 3.7, 7.5, 22.7 us; 30000 rows,
-// K = 1024, 8 rows: 66.9 -> 15.2 us (4.0 TB/s).
+// K = 1024, 8 rows: 66.9 -> 15.2 us (4.0 TB/s). Those read one matrix over and
+// over; between the other kernels of a layer the router takes 4.5 and 8.7 us at 4
+// and 512 rows.
 template <int MT, int R>
 __global__ __launch_bounds__(256) void gemv_dense_bf16(DenseOp op) {
     __shared__ float part[4][R][MT];

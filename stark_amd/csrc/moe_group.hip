@@ -10,8 +10,9 @@
 // groups are one v_mfma_f32_16x16x4_f32 (f32 products and sums).
 //
 // What bounds it: at 512 tokens (32 routes an expert on average) the 340 MB of
-// expert weights; the matrix and vector work of 64 routes takes about as long
-// as the workgroup's share of the HBM rate. Hence:
+// expert weights are 60 us of HBM and take 132: the vector work of a group (the
+// exponents, the scaling of every sum) beside the loads, most of all in the up
+// product, whose activations every column tile converts again. Hence:
 //  - B operands come straight from global memory: a lane loads 16 bytes (32
 //    codes) of its row, so an instruction reads 64 bytes of each of 16 rows,
 //    and v_permlane32_swap sorts the words so that all four lane groups of an
@@ -27,11 +28,10 @@
 //    in flight.
 // Measured (model 2048, hidden 768, 128 experts, top 8, router included): 512
 // tokens 1978 -> 178 us, 160 with the router's later product (the products
-// 1103 + 851 -> 86 + 46 us, 4.0 and 2.5 TB/s of weights); 30 tokens over 96
-// experts: the up product 5.2 TB/s. The
-// slot form of mfma_tile.h (16 routes a slot, half of every MFMA empty, codes
-// through LDS, the weights once per 16 routes) stays for group sizes 32 and
-// 128 and for at most 16 tokens.
+// 1103 + 851 -> 86 + 46 us, 2.6 and 2.5 TB/s of weights). The slot form of
+// mfma_tile.h (16 routes a slot, half of every MFMA empty, codes through LDS, the
+// weights once per 16 routes) stays for group sizes 32 and 128 and where
+// moe_grouped (dispatch_rules.h) says so.
 #include "qmm_common.h"
 #include "code_layout.h"
 
@@ -59,34 +59,11 @@ struct GroupLds {
     uint32_t route[kSlot];
 };
 
-__device__ __forceinline__ uint32_t permb(uint32_t hi, uint32_t lo, uint32_t sel) {
-    return __builtin_amdgcn_perm(hi, lo, sel);
-}
-
-// silu(gate) * value in bf16 steps (gated_act_mul; SiLU as
-// src/backends/common/gpu_types/activation_type.rs:35-46)
-__device__ __forceinline__ uint16_t gated(float value_f, float gate_f) {
-    const float v = bf16_bits_to_f32(f32_to_bf16_bits(value_f));
-    const float x = bf16_bits_to_f32(f32_to_bf16_bits(gate_f));
-    const float y = x / (1.0f + expf(-1.0f * x));
-    const float a = bf16_bits_to_f32(f32_to_bf16_bits(y));
-    return f32_to_bf16_bits(v * a);
-}
-
 // B operand (8 codes of one row) of a code word: pairs (q0, q4) (16 q1, 16 q5)
 // (q2, q6) (16 q3, 16 q7), as the activations are staged.
 __device__ __forceinline__ bf16x8 codes8(uint32_t u) {
     const uint32_t v = u >> 8;
     return __builtin_bit_cast(bf16x8, u32x4{u & 0x000F000Fu, u & 0x00F000F0u, v & 0x000F000Fu, v & 0x00F000F0u});
-}
-
-// MFMA order of the 8-value pieces of a 64-value group: the lane of k quarter
-// kq takes piece 4 (kq & 1) + 2 j + (kq >> 1) for the group's j-th MFMA (what
-// permlane32_swap makes of 16-byte code loads), so piece v is stored at
-// 4 j + kq with j = (v >> 1) & 1 and kq = (v >> 2) | 2 (v & 1).
-__device__ __forceinline__ uint32_t piece_pos(uint32_t v) {
-    const uint32_t g = v >> 3, p = v & 7;
-    return 8 * g + 4 * ((p >> 1) & 1) + ((p >> 2) | ((p & 1) << 1));
 }
 
 // One column tile of one slot with MT 16-row blocks of routes. UP: the waves'
@@ -167,7 +144,7 @@ __device__ __forceinline__ void group_tile(const MoeGroup& L, GroupLds& lds, uin
             q[1] = permb(__float_as_uint(f[5]), __float_as_uint(f[1]), 0x07060302u);
             q[2] = permb(__float_as_uint(f[6]), __float_as_uint(f[2]), 0x07060302u);
             q[3] = permb(__float_as_uint(f[7]), __float_as_uint(f[3]), 0x07060302u);
-            lds.xa[buf][piece_pos(piece) * kRowPad + r] = q;
+            lds.xa[buf][piece_pos<4>(piece) * kRowPad + r] = q;
             float sm = 0.0f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) sm = dot2_bf16(t[e], 0x3F803F80u, sm);
@@ -245,11 +222,6 @@ __device__ __forceinline__ void group_tile(const MoeGroup& L, GroupLds& lds, uin
                 acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs, bt[t], acc[m][t], 0, 0, 0);
         }
     };
-    const auto lds_barrier = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
 
     // Chunk c computes from LDS buffer c % 2 and code set c % 2. The prefetches
     // past the last chunk are clamped to it (their buffers are not computed).
@@ -291,7 +263,7 @@ __device__ __forceinline__ void group_tile(const MoeGroup& L, GroupLds& lds, uin
             if (r >= cnt) continue;
             uint16_t* o = L.out + (size_t)lds.route[r] * N + n0 + col;
             if (UP) {
-                o[0] = gated(acc[m][0][e], acc[m][1][e]);
+                o[0] = gated_silu(acc[m][0][e], acc[m][1][e]);
             } else {
                 o[0] = f32_to_bf16_bits(acc[m][0][e]);
                 o[16] = f32_to_bf16_bits(acc[m][1][e]);

@@ -309,16 +309,6 @@ __device__ __host__ inline uint32_t line_tiles(uint32_t tiles, uint32_t rows) {
     return tiles % tpl == 0 ? tpl : 1u;
 }
 
-// silu(gate) * value in bf16 steps (gated_act_mul; SiLU as
-// src/backends/common/gpu_types/activation_type.rs:35-46)
-__device__ __forceinline__ uint16_t gated_silu(float value_f, float gate_f) {
-    const float v = bf16_bits_to_f32(f32_to_bf16_bits(value_f));
-    const float x = bf16_bits_to_f32(f32_to_bf16_bits(gate_f));
-    const float y = x / (1.0f + expf(-1.0f * x));
-    const float a = bf16_bits_to_f32(f32_to_bf16_bits(y));
-    return f32_to_bf16_bits(v * a);
-}
-
 // ---- 3. grouped up product + gated SiLU. Work item = (slot, tile of 8 value rows).
 template <int MP, int MB, int GS, bool SIGNED, int P1>
 __global__ __launch_bounds__(kWg) void moe_up_mfma(GroupedLaunch launch) {

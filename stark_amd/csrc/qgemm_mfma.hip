@@ -238,11 +238,6 @@ __device__ __forceinline__ void gemm_tile(const AffineOp& op, uint32_t bx, uint3
     // (loaded NS - 1 steps earlier) is dequantised into the other buffer and
     // the loads of steps s+2 .. s+NS fly; the barriers order LDS only, so
     // those loads stay in flight across them.
-    const auto lds_barrier = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
     const uint32_t steps = K / kBK;
     // Branch-free body (a conditional load would make the compiler wait for
     // every load before the next dequantisation): the step indices of the

@@ -197,11 +197,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             }
         }
     };
-    const auto lds_barrier = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
 
     // Pass q multiplies LDS buffer q % 2; prefetches past the last pass are
     // clamped to it (what they bring is not computed). PIPE: the operands of pass

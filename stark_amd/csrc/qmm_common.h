@@ -49,6 +49,25 @@ QMM_DEVICE void store_from_f32(void* p, uint32_t dt, size_t i, float v) {
     }
 }
 
+// silu(gate) * value in bf16 steps (gated_act_mul; SiLU as
+// src/backends/common/gpu_types/activation_type.rs:35-46)
+QMM_DEVICE uint16_t gated_silu(float value_f, float gate_f) {
+    const float v = bf16_bits_to_f32(f32_to_bf16_bits(value_f));
+    const float x = bf16_bits_to_f32(f32_to_bf16_bits(gate_f));
+    const float y = x / (1.0f + expf(-1.0f * x));
+    const float a = bf16_bits_to_f32(f32_to_bf16_bits(y));
+    return f32_to_bf16_bits(v * a);
+}
+
+QMM_DEVICE uint32_t permb(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
+
+// Workgroup barrier that orders LDS only: global loads stay in flight across it.
+QMM_DEVICE void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Full 64-lane sum; every lane receives the total.
 QMM_DEVICE float wave_sum(float v) {
 #pragma unroll

@@ -256,11 +256,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             for (int t = 0; t < 2; ++t) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u, bt[t], acc[m][t], 0, 0, 0);
         }
     };
-    const auto lds_barrier = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
     const auto groups = [&](uint32_t p) -> uint32_t {
         const uint32_t g = p * kGroups + 2 * kw;
         return g + 2 <= G ? 2u : g < G ? 1u : 0u;

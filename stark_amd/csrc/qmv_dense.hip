@@ -48,20 +48,6 @@ struct DenseLds {
     uint32_t pl[2][kThreads];  // raw scale | bias << 16, [group][column]
 };
 
-__device__ __forceinline__ uint32_t permb(uint32_t hi, uint32_t lo, uint32_t sel) {
-    return __builtin_amdgcn_perm(hi, lo, sel);
-}
-
-// Place of 8-value piece v of a pass in MFMA order. 4-bit: within a 64-value
-// group, piece 4 (kq & 1) + 2 j + (kq >> 1) belongs to lane quarter kq of the
-// group's j-th MFMA (what permlane32_swap makes of 16-byte loads); 8-bit: piece
-// 2 kq + j.
-template <int BITS>
-__device__ __forceinline__ uint32_t piece_pos(uint32_t v) {
-    const uint32_t p = v & 7;
-    return (v & ~7u) + (BITS == 4 ? 4 * ((p >> 1) & 1) + ((p >> 2) | ((p & 1) << 1)) : 4 * (p & 1) + (p >> 1));
-}
-
 template <int BITS, int EM, bool BIASED, bool BF>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 1 ? 5 : 4))) void qmv_dense(
     AffineBatch batch) {
@@ -235,11 +221,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 
 #pragma unroll
             for (int e = 0; e < EM; ++e) asm volatile("" : "+v"(acc[0][e]), "+v"(acc[1][e]));
         }
-    };
-    const auto lds_barrier = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
     // groups of this wave's chunk in a pass
     const auto groups = [&](uint32_t p) -> uint32_t {

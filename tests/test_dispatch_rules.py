@@ -7,6 +7,7 @@ from tests import dispatch as D
 from tests import helpers as H
 from tests import test_gpu_a8_dense as A8
 from tests import test_gpu_affine_dense as AD
+from tests import test_gpu_exact_dequant as ED
 from tests import test_gpu_gemm_stream as GS
 from tests import test_gpu_moe_group as MG
 from tests import test_gpu_small_m as SM
@@ -175,3 +176,5 @@ def test_stream_cases_reach_both_widths_and_the_kernel():
     for m, n, k in GS.EXACT:
         assert m <= 64 or (D.stream_takes([(m, n, k)], 4) and D.stream_takes([(m, n, k)], 8)), (m, n, k)
     assert {D.stream_blocks([(m, n, k)]) for m, n, k in GS.EXACT} == {2, 3, 4}
+    for bits in (4, 8):
+        assert not D.stream_takes([ED.GEMM64 + (64,)], bits) and not D.stream_takes([ED.GEMM64 + (704,)], bits)

@@ -578,9 +578,8 @@ def test_prefill_gemm_full_width(qmm, oracle):
                                    (130, 1000, 192)])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_prefill_gemm_shapes(qmm, oracle, m, n, k, bits):
-    """M > 16 runs the matrix-core dequant-GEMM (4-bit g64 products of at most
-    32 rows with K % 512 == 0 the skinny product, same arithmetic):
-    bf16-effective weights, f32 accumulation. Checked against the f64 product of the same bf16 weights, and
+    """M > 16 runs the matrix-core dequant-GEMM (up to 128 rows qgemm_stream,
+    the same arithmetic): bf16-effective weights, f32 accumulation. Checked against the f64 product of the same bf16 weights, and
     against the exact-f32 CPU kernel at the reference's own GPU/CPU bar
     (quant_dispatch_test.rs:189: rel 0.05 / abs 0.4)."""
     rng = np.random.default_rng(m * 7 + n + bits)
@@ -608,10 +607,10 @@ def test_prefill_gemm_shapes(qmm, oracle, m, n, k, bits):
     assert np.all(np.abs(got.ravel() - exact) <= 0.05 * np.abs(exact) + 0.4)
 
 
-def _skinny_case(qmm, oracle, m, n, k, *, layout=1, correction=1, signed=False, w_dt=H.BF16, seed=0, d_dt=H.F32,
+def _short_prompt_case(qmm, oracle, m, n, k, *, layout=1, correction=1, signed=False, w_dt=H.BF16, seed=0, d_dt=H.F32,
                  ab_scale=1.0, accumulate=False, with_bias=False, soft_cap=None):
-    """A 4-bit g64 product of 17 .. 32 rows (the skinny product) against the
-    f64 product of the bf16-effective weights, at the prefill bar."""
+    """A 4-bit g64 product of 17 rows and more against the f64 product of the
+    bf16-effective weights, at the prefill bar."""
     rng = np.random.default_rng(seed)
     W = H.affine_weights(oracle, rng, n, k, 4, 64, layout, correction, w_dt)
     x = H.activations(oracle, rng, m, k, H.BF16)
@@ -637,33 +636,31 @@ def _skinny_case(qmm, oracle, m, n, k, *, layout=1, correction=1, signed=False, 
     if soft_cap is not None:
         want = soft_cap * np.tanh(want / soft_cap)
     check(got.ravel(), want.ravel(), mag=(mag * abs(ab_scale) + (4.0 if accumulate else 0.0)).ravel(),
-          label=f"skinny m{m} n{n} k{k}")
+          label=f"short prompt m{m} n{n} k{k}")
 
 
 @pytest.mark.parametrize("m,n,k", [(17, 16, 512), (24, 40, 1536), (32, 1000, 4096), (20, 9000, 4096),
                                    (32, 96, 12288), (31, 32010, 512), (33, 72, 1024), (48, 1000, 4096),
                                    (64, 9000, 4096)])
 @pytest.mark.parametrize("layout", [0, 1])
-def test_skinny_product_shapes(qmm, oracle, m, n, k, layout):
-    """17 .. 64 rows, 4-bit g64, K % 512 == 0: the skinny product (one tile
-    pair; ragged N; runs of several pairs at N = 9000 and 32010; deep K;
-    33 .. 64 rows as two 32-row blocks, the second one short)."""
-    _skinny_case(qmm, oracle, m, n, k, layout=layout, seed=m + n + k + layout)
+def test_short_prompt_shapes(qmm, oracle, m, n, k, layout):
+    """17 .. 64 rows, 4-bit g64, on qgemm_stream: half a tile of columns,
+    ragged N, many columns (N = 9000 and 32010, both widths), deep K."""
+    _short_prompt_case(qmm, oracle, m, n, k, layout=layout, seed=m + n + k + layout)
 
 
 @pytest.mark.parametrize("variant", ["symmetric", "signed", "signed_symmetric", "f16_planes", "bf16_out", "d_ops"])
-def test_skinny_product_variants(qmm, oracle, variant):
+def test_short_prompt_variants(qmm, oracle, variant):
     kw = {"symmetric": dict(correction=0), "signed": dict(signed=True),
           "signed_symmetric": dict(correction=0, signed=True),
           "f16_planes": dict(w_dt=H.F16), "bf16_out": dict(d_dt=H.BF16),
           "d_ops": dict(ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=30.0)}[variant]
-    _skinny_case(qmm, oracle, 27, 9000, 4096, seed=400 + len(variant), **kw)
+    _short_prompt_case(qmm, oracle, 27, 9000, 4096, seed=400 + len(variant), **kw)
 
 
-def test_skinny_product_batch_matches_single(qmm, oracle):
-    """A K = 12288 and a K = 4096 product of 32 rows in one launch (one pair
-    per workgroup) give the bits of two single launches (three pairs per
-    workgroup for the K = 4096 one)."""
+def test_short_prompt_batch_matches_single(qmm, oracle):
+    """A K = 12288 and a K = 4096 product of 32 rows in one launch give the
+    bits of two single launches."""
     rng = np.random.default_rng(41)
     k = qmm.MatmulKernel(H.BF16, H.BF16, H.BF16)
     made = []
@@ -689,8 +686,8 @@ def test_skinny_product_batch_matches_single(qmm, oracle):
 
 def test_encode_many_mixed_row_classes_match_single(qmm, oracle):
     """One encode_many call over products of 1, 2, 8, 24, 48 and 100 rows (the
-    streaming kernel, the slot form, the small-M kernel, both skinny classes
-    and the GEMM) gives each product the bits of its own encode call."""
+    decode stream, the slot form, the dense kernel and three row blocks of
+    qgemm_stream) gives each product the bits of its own encode call."""
     rng = np.random.default_rng(43)
     k = qmm.MatmulKernel(H.BF16, H.BF16, H.BF16)
     made = []
@@ -752,7 +749,7 @@ def test_encode_many_row_classes_in_graph_replays(qmm, oracle):
 
 @pytest.mark.parametrize("correction,signed,w_dt,gs", [(0, False, H.BF16, 64), (1, True, H.F16, 32),
                                                        (0, True, H.BF16, 128), (1, False, H.F16, 64)])
-@pytest.mark.parametrize("m", [40, 200])  # 40: skinny (group 64) or 128x64 GEMM tiles; 200: 128x128 tiles
+@pytest.mark.parametrize("m", [40, 200])  # 40: qgemm_stream (group 64) or 128x64 GEMM tiles; 200: 128x128 tiles
 def test_prefill_gemm_corrections(qmm, oracle, correction, signed, w_dt, gs, m):
     n, k = 160, 512
     rng = np.random.default_rng(gs + correction)

@@ -247,7 +247,7 @@ def _gemm_exact(Q, O, *, n, k, bits, correction=1, signed=False, layout=0, seed=
     gs = 64
     codes, s, b = _weights(O, rng, n, k, bits, gs, layout, correction, H.BF16)
     cols = _columns(rng, k, 40)
-    cols = np.resize(cols, m)  # M > 64 takes the GEMM, 17 .. 64 (4-bit g64, K % 512 == 0) the skinny product
+    cols = np.resize(cols, m)
     x = H.store(O, _one_hot(k, cols, H.BF16).ravel(), H.BF16)
     G = k // gs
     if correction == 1 and not signed and bits in (4, 8):
@@ -291,26 +291,35 @@ def test_gemm_exact_variants(qmm, oracle, correction, signed):
                                  (72, 3136), (385, 448), (520, 320)])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_gemm_exact_tile_classes(qmm, oracle, m, k, bits):
-    """The three GEMM tile classes (128x64 tiles up to 128 rows, 128x128 up
-    to 384, both of eight waves with three load stages; 256x128 above) at
-    64-value step counts that leave every remainder of the six-step unrolled
-    blocks (1, 6 .. 11 and 49 steps; odd and even counts in the 256-row
-    class), ragged N: the bf16 weight tiles stay bit-exact."""
+    """Two GEMM tile classes (128x128 up to 384 rows, of eight waves with three
+    load stages; 256x128 above) at 64-value step counts that leave every
+    remainder of the six-step unrolled blocks (1, 6 .. 11 and 49 steps; odd and
+    even counts in the 256-row class), ragged N, and qgemm_stream up to 128
+    rows of these few columns: the bf16 weight tiles stay bit-exact."""
     _gemm_exact(qmm, oracle, n=136, k=k, bits=bits, seed=200 + m + bits, m=m)
+
+
+GEMM64 = (97, 8260)  # rows, columns: more than the rule leaves to qgemm_stream
+
+
+@pytest.mark.parametrize("k", [64, 128, 448, 512, 576, 640, 704])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_gemm_exact_64_column_tiles(qmm, oracle, k, bits):
+    """The third class, 128x64 tiles (eight waves, three load stages), at the same remainders."""
+    _gemm_exact(qmm, oracle, n=GEMM64[1], k=k, bits=bits, layout=k // 64 % 2, seed=230 + k + bits, m=GEMM64[0])
 
 
 @pytest.mark.parametrize("m", [17, 32, 40])
 @pytest.mark.parametrize("layout", [0, 1])
-def test_skinny_exact_against_bf16_effective_oracle(qmm, oracle, m, layout):
-    """qgemm_skinny (4-bit, 17 .. 64 rows; 40 rows as blocks of 32 and 8)
-    dequantises to the same bf16 weights as the GEMM, bit for bit."""
-    _gemm_exact(qmm, oracle, n=96, k=512, bits=4, layout=layout, seed=190 + m + layout, m=m, label="qgemm_skinny")
+def test_stream_exact_against_bf16_effective_oracle(qmm, oracle, m, layout):
+    """qgemm_stream (blocks of 32 and 48 rows) dequantises to the same bf16 weights as the GEMM, bit for bit."""
+    _gemm_exact(qmm, oracle, n=96, k=512, bits=4, layout=layout, seed=190 + m + layout, m=m, label="qgemm_stream")
 
 
 @pytest.mark.parametrize("correction,signed", [(0, False), (1, True), (0, True)])
-def test_skinny_exact_variants(qmm, oracle, correction, signed):
+def test_stream_exact_variants(qmm, oracle, correction, signed):
     _gemm_exact(qmm, oracle, n=48, k=1024, bits=4, correction=correction, signed=signed, seed=195 + correction,
-                m=24, label="qgemm_skinny")
+                m=24, label="qgemm_stream")
 
 
 # ------------------------------------------------------------ GGUF blocks (hybrid path)

@@ -40,7 +40,7 @@ def test_stream_corrections_exact(qmm, oracle, correction, signed, bits, m):
 @pytest.mark.parametrize("m,n,k,f16,wide", SUMS)
 def test_stream_sums(qmm, oracle, m, n, k, f16, wide):
     """Both column widths against the f64 product of the bf16-effective weights, with the D-ops; f16 planes and results at two sizes."""
-    A._skinny_case(qmm, oracle, m, n, k, seed=m + n, ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=30.0,
+    A._short_prompt_case(qmm, oracle, m, n, k, seed=m + n, ab_scale=0.75, accumulate=True, with_bias=True, soft_cap=30.0,
                    w_dt=H.F16 if f16 else H.BF16, d_dt=H.BF16 if f16 else H.F32)
 
 
