@@ -146,11 +146,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 
         lds.pl[buf][pg * kCols + pc] = ps | (pb << 16);
     };
 
-    float acc[2][EM];
+    // The f32 error comes from the running sums' roundings, two a group (K 12288,
+    // 4-bit, 12 rows: 1.62e-7 of the result, 8-bit 1.61e-7): two sums (1.38e-7,
+    // within 0.5% of the time), or, for 8-bit rows 9 to 16, whose second sums
+    // spill (+7%), one that takes a group's two terms joined (1.35e-7, +1%; joined
+    // everywhere: +1% everywhere).
+    constexpr int SUMS = BITS == 8 && EM == 4 ? 1 : 2;
+    float acc[SUMS][2][EM];  // [group of a chunk][tile][entry]
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int g = 0; g < SUMS; ++g)
 #pragma unroll
-        for (int e = 0; e < EM; ++e) acc[t][e] = 0.0f;
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < EM; ++e) acc[g][t][e] = 0.0f;
     // this lane's A row: MFMA row col = 4 (r % 4) + r / 4; entries past EM repeat a row and are not read
     const uint32_t arow = (col >> 2) + ((col & 3) < (uint32_t)EM ? 4 * (col & 3) : 0);
     const auto compute = [&](int buf, u32x4 (&w)[2][WL], uint32_t ng) {
@@ -214,12 +222,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 
                                  : BF    ? __uint_as_float(p & 0xffff0000u)
                                          : f16_bits_to_f32(p >> 16);
 #pragma unroll
-                for (int e = 0; e < EM; ++e)
-                    acc[t][e] = fmaf(sc, ldexp_f32(c[e], xg[e].e), fmaf(bi, xg[e].sum, acc[t][e]));
+                for (int e = 0; e < EM; ++e) {
+                    float& s = acc[g % SUMS][t][e];
+                    const float d = ldexp_f32(c[e], xg[e].e);
+                    s = SUMS == 2 ? fmaf(sc, d, fmaf(bi, xg[e].sum, s)) : s + fmaf(sc, d, bi * xg[e].sum);
+                }
             }
             // keeps the scaling here: moved past the staging and the barrier, it would hold every group's sums live
 #pragma unroll
-            for (int e = 0; e < EM; ++e) asm volatile("" : "+v"(acc[0][e]), "+v"(acc[1][e]));
+            for (int e = 0; e < EM; ++e) asm volatile("" : "+v"(acc[g % SUMS][0][e]), "+v"(acc[g % SUMS][1][e]));
         }
     };
     // groups of this wave's chunk in a pass
@@ -262,7 +273,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(EM == 
 #pragma unroll
         for (int e = 0; e < EM; ++e) {
             const uint32_t r = kq + 4 * e;
-            lds.red[(wave * R + r) * kCols + 16 * t + col] = acc[t][e];
+            lds.red[(wave * R + r) * kCols + 16 * t + col] = SUMS == 2 ? acc[0][t][e] + acc[1][t][e] : acc[0][t][e];
         }
     lds_barrier();
     for (uint32_t q = tid; q < M * kCols; q += kThreads) {
