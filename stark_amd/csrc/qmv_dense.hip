@@ -337,24 +337,33 @@ DenseRule::DenseRule(const AffineOp* ops, uint32_t count, int b)
         if (dense_eligible(ops[0], bits)) few_rows = few_rows_rule(ops, 1, bits, 0u, readable);
         return;
     }
-    std::vector<AffineOp> few, mid, many;
-    bool mid_readable = true;
-    for (uint32_t i = 0; i < count; ++i) {
-        const AffineOp& o = ops[i];
-        if (!dense_eligible(o, bits)) continue;
-        if (o.m <= 2) {
-            few.push_back(o);
-        } else if (o.m > 8) {
-            if (bits == 4) many.push_back(o);
-        } else if (o.m > 4 && bits == 8) {
-            mid.push_back(o);
-            mid_readable = mid_readable && readable(o);
-        }
+    // the products of each rule: the call's own array where they all fall under one
+    const auto rule_of = [&](const AffineOp& o) {
+        if (!dense_eligible(o, bits)) return 0;
+        if (o.m <= 2) return 1;
+        if (o.m > 8) return bits == 4 ? 2 : 0;
+        return o.m > 4 && bits == 8 ? 3 : 0;
+    };
+    uint32_t n[4] = {};
+    for (uint32_t i = 0; i < count; ++i) ++n[rule_of(ops[i])];
+    std::vector<AffineOp> part;
+    const auto products = [&](int rule) {
+        if (n[rule] == count) return ops;
+        part.clear();
+        part.reserve(n[rule]);
+        for (uint32_t i = 0; i < count; ++i)
+            if (rule_of(ops[i]) == rule) part.push_back(ops[i]);
+        return (const AffineOp*)part.data();
+    };
+    if (n[1]) few_rows = few_rows_rule(products(1), n[1], bits, cus(), readable);
+    if (n[2]) {
+        const AffineOp* many = products(2);
+        if (small_m_eligible(many, n[2])) many_rows = !small_m_long(many, n[2], cus());
     }
-    if (!few.empty()) few_rows = few_rows_rule(few.data(), (uint32_t)few.size(), bits, cus(), readable);
-    if (!many.empty() && small_m_eligible(many.data(), (uint32_t)many.size()))
-        many_rows = !small_m_long(many.data(), (uint32_t)many.size(), cus());
-    if (!mid.empty() && mid_readable) mid_rows = !w8_rows5_mfma(mid.data(), (uint32_t)mid.size(), cus());
+    if (n[3]) {
+        const AffineOp* mid = products(3);
+        if (std::all_of(mid, mid + n[3], readable)) mid_rows = !w8_rows5_mfma(mid, n[3], cus());
+    }
 }
 
 bool DenseRule::takes(const AffineOp& o) const {
